@@ -1501,8 +1501,8 @@ __global__ __launch_bounds__(1024) void paged_decode_split_combine_kernel(const 
 // ------------------------------------------------------------------------------ row-parallel path
 // Narrow tables (at most kMaxRowTiles tiles of capacity per row, any batch) and small batches (at most
 // kRowMaxBatch rows, up to kRowMaxWaves * kRowMaxPer tiles): one workgroup per (row, KV head) whose W waves take
-// the row's tiles round-robin (W = the capacity in tiles up to 16, else 8; wave w streams tiles w, w + W, ..., lane i
-// of its list describing tile w + i*W), so a row's tiles are spread over up to 16 waves instead of a chain of
+// the row's tiles round-robin (W = the capacity in tiles up to 8; wave w streams tiles w, w + W, ..., lane i
+// of its list describing tile w + i*W), so a row's tiles are spread over up to 8 waves instead of a chain of
 // workgroups and a combine.  Everything that does not depend on the context is loaded at once: the row's context,
 // the wave's table entries (entries past the context are read but never used), q, and in the append form the new
 // k/v rows (parked in the wave's LDS until the tile that needs them); with one tile per wave (kMulti false) the
@@ -1514,9 +1514,10 @@ constexpr int kRowMaxWaves = 16;
 constexpr int kRowMaxPer = 8;             // rows of up to kRowMaxWaves * kRowMaxPer tiles = 2,048 tokens
 constexpr int kRowMaxBatch = 64;            // beyond, stream-K (equal at 128-256 rows, ahead when ragged)
 constexpr int kRowRec = kG * kD + 2 * kG;  // floats per wave state: acc[kG][kD], m[kG], l[kG]
-// With several tiles per wave the append form needs more than the 128 registers a 16-wave workgroup allows, so both
-// forms then run 8 waves of up to 16 tiles (the same decomposition: the append form stays bitwise equal to a scatter
-// followed by the plain form).
+// With several tiles per wave a workgroup has 8 waves of up to 16 tiles, and two workgroups share a CU: the new token's
+// swap is pinned ahead of the tile's arithmetic, which keeps the append forms at 116 registers (147 left to itself: one
+// workgroup a CU).  64 rows log-uniform in [64, 1200]: 30.2 -> 25.2 us per call with the head-fastest grid; 20 rows of
+// up to 60 tokens in 256-token tables, 16 waves of one tile -> 8 of two: 8.1 -> 5.7.
 constexpr int row_max_waves(bool multi) { return multi ? kRowMaxWaves / 2 : kRowMaxWaves; }
 
 //
@@ -1527,20 +1528,78 @@ constexpr int row_max_waves(bool multi) { return multi ? kRowMaxWaves / 2 : kRow
 // state (fp32 o = sum p.v, m, l of both query heads) as a record, which paged_decode_chunk_combine_kernel merges.
 constexpr int kChunkMax = 16;  // records per (row, KV head): the combine loads them all at once
 
-template <bool kAppend, bool kMulti, bool kRope = false>
-__global__ __launch_bounds__(64 * row_max_waves(kMulti)) void paged_decode_row_kernel(const DecodeArgs a) {
+//
+// Balanced form (kBal), for kBalMinBatch..kBalMaxBatch rows: the chunks are cut from the lengths the call finds on
+// the device, not from the table capacity.  Each workgroup (4 waves) loads every row's length (one lane a row), derives
+// the same chunk length from their total, so that the rows' chunks together are about the workgroups the device
+// holds at once.  Workgroup b < batch takes row b's first chunk and loads its table entries and q beside the lengths;
+// the others find their (row, chunk >= 1) by a scan and a ballot, one more round trip, or exit past the last one.
+constexpr int kBalWaves = 4;
+
+struct BalSplit {
+  int ctx, n, nch;  // lane i: row i's context, tiles and chunks (at least 1 for a row of the batch: it writes zeros)
+};
+
+// The rows' cache_seqlens, lane i row i's (past the batch: the last row's, which balanced_split drops).
+__device__ __forceinline__ int balanced_seqlens(const DecodeArgs& a, int lane) { return a.seqlens[min(lane, a.batch - 1)]; }
+
+// ceil(n / d) for 0 <= n < 2^20, 1 <= d: the quotient is at least 1 / (2 d) away from the next integer, far more than
+// the reciprocal's error.
+__device__ __forceinline__ int ceil_div_small(int n, int d) {
+  return (int)(((float)(n + d) - 0.5f) * __builtin_amdgcn_rcpf((float)d));
+}
+
+template <bool kAppend>
+__device__ __forceinline__ BalSplit balanced_split(const DecodeArgs& a, int c, int lane) {
+  BalSplit s;
+  s.ctx = lane < a.batch ? ctx_of<kAppend>(c, a.max_pages * a.page_size) : 0;
+  s.n = (s.ctx + kTile - 1) / kTile;
+  const int total = readlane(wave_scan_incl(s.n), 63);
+  const int ct = max(a.row_per, __builtin_amdgcn_readfirstlane(ceil_div_small(total, a.grid)));
+  s.nch = lane < a.batch ? max(1, ceil_div_small(s.n, ct)) : 0;
+  return s;
+}
+
+template <bool kAppend, bool kMulti, bool kRope = false, bool kBal = false>
+__global__ __launch_bounds__(64 * (kBal ? kBalWaves : row_max_waves(kMulti)), kBal ? 4 : 1)
+void paged_decode_row_kernel(const DecodeArgs a) {
   static_assert(kAppend || !kRope, "the norm/rope form is an append form");
-  __shared__ __align__(16) float rec[kRowMaxWaves][kRowRec];
-  __shared__ __align__(16) uint4 snew[kAppend ? kRowMaxWaves : 1][2][kD / 8];  // per wave: the new k and v rows
-  const int b = blockIdx.x;
-  const int g = blockIdx.y;
+  constexpr int kWaves = kBal ? kBalWaves : kRowMaxWaves;
+  __shared__ __align__(16) float rec[kWaves][kRowRec];
+  __shared__ __align__(16) uint4 snew[kAppend ? kWaves : 1][2][kD / 8];  // per wave: the new k and v rows
+  // The KV head is the fastest grid dimension: workgroups go to the XCDs in launch order, so with 8 heads every XCD
+  // reads one head of every row.  With the row fastest, rows b, b + 8, ... shared an XCD, and the XCD with the
+  // longest rows decided the call.
+  const int g = blockIdx.x;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int W = (int)(blockDim.x >> 6);
+  const int W = kBal ? kBalWaves : (int)(blockDim.x >> 6);
   const int lane = threadIdx.x & 63;
   const int grp = lane >> 4;
   const int dl = (lane & 15) * 8;
-  const int CT = W * a.row_per;              // tiles per chunk (the one-launch path: the whole table)
-  const int tb = (int)blockIdx.z * CT;       // first tile of this workgroup's chunk
+  int b = blockIdx.y, ch = 0, CT = 0, ctx = 0, nch = 0;  // row, chunk, tiles per chunk, the row's context and chunks
+  int c_row = 0;
+  // Row r's context, chunks and (equal) chunk length from the split of all rows.
+  auto take = [&](const BalSplit& s, int r) __attribute__((always_inline)) {
+    ctx = readlane(s.ctx, r);
+    nch = readlane(s.nch, r);
+    CT = max(1, __builtin_amdgcn_readfirstlane(ceil_div_small(readlane(s.n, r), nch)));
+  };
+  if constexpr (kBal) {
+    c_row = balanced_seqlens(a, lane);
+    if (b >= a.batch) {
+      const int extra = b - a.batch;  // this workgroup's place among the rows' chunks 1, 2, ...
+      const BalSplit s = balanced_split<kAppend>(a, c_row, lane);
+      const int incl = wave_scan_incl(max(s.nch - 1, 0));
+      if (extra >= readlane(incl, 63)) return;  // uniform over the workgroup
+      b = __builtin_popcountll(__ballot(incl <= extra));
+      take(s, b);
+      ch = extra - (readlane(incl, b) - nch);
+    }
+  } else {
+    ch = blockIdx.z;
+    CT = W * a.row_per;  // the one-launch path: the whole table
+  }
+  const int tb = ch * CT;  // first tile of this workgroup's chunk
 
   // Every load that does not depend on the context goes out together with the row's cache_seqlens entry: the
   // table entry of this lane's tile, q, (append form) the new k/v rows, (norm/rope form) the weights and cos/sin.
@@ -1550,7 +1609,7 @@ __global__ __launch_bounds__(64 * row_max_waves(kMulti)) void paged_decode_row_k
   __asm__ volatile("" ::"s"(a.seqlens), "s"(a.bt), "s"(a.bt_sb), "s"(a.max_pages), "s"(a.page_size), "s"(a.row_per),
                    "s"(a.q), "s"(a.q_sb), "s"(a.q_sh), "s"(a.scale_log2), "s"(a.kc), "s"(a.vc), "s"(a.kv_sp),
                    "s"(a.kv_st), "s"(a.kv_sh));
-  const int c_row = a.seqlens[b];
+  if constexpr (!kBal) c_row = a.seqlens[b];
   const int cap = a.max_pages * a.page_size;
   const int t = kTile * (tb + w + lane * W);  // first token of this lane's tile
   const int pidx = min(t, cap - 1) / a.page_size;
@@ -1581,12 +1640,16 @@ __global__ __launch_bounds__(64 * row_max_waves(kMulti)) void paged_decode_row_k
       snew[w][1][lane] = vn;
     }
   }
-  const int ctx = ctx_of<kAppend>(c_row, cap);
+  if constexpr (kBal) {
+    if (ch == 0) take(balanced_split<kAppend>(a, c_row, lane), b);
+  } else {
+    ctx = ctx_of<kAppend>(c_row, cap);
+  }
   const int nrow = (ctx + kTile - 1) / kTile;  // tiles of the row
-  const int nch = (nrow + CT - 1) / CT;        // chunks holding tiles of the row
+  if constexpr (!kBal) nch = (nrow + CT - 1) / CT;  // chunks holding tiles of the row
   // Chunks past the row's end have nothing to do (chunk 0 stays: it writes the zero row of an empty one).  The
   // condition is uniform over the workgroup.
-  if (blockIdx.z > 0 && (int)blockIdx.z >= nch) return;
+  if (!kBal && ch > 0 && ch >= nch) return;
   const int nrc = min(nrow - tb, CT);          // tiles of the row in this chunk
 
   TileList L;
@@ -1611,16 +1674,16 @@ __global__ __launch_bounds__(64 * row_max_waves(kMulti)) void paged_decode_row_k
     if constexpr (kAppend) {
       if (j == jt) {
         const int tn = readlane(L.nvalid, j) - 1;
-        const uint4 kn = snew[w][0][lane & 15];
-        const uint4 vn = snew[w][1][lane & 15];
+        const uint4 kn = ld16(&snew[w][0][lane & 15]);
+        const uint4 vn = ld16(&snew[w][1][lane & 15]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          if (i == (tn >> 2) && grp == (tn & 3)) {
-            T.k[i] = kn;
-            T.v[i] = vn;
-          }
+          const bool mine = 4 * i + grp == tn;
+          T.k[i] = make_uint4(mine ? kn.x : T.k[i].x, mine ? kn.y : T.k[i].y, mine ? kn.z : T.k[i].z, mine ? kn.w : T.k[i].w);
+          T.v[i] = make_uint4(mine ? vn.x : T.v[i].x, mine ? vn.y : T.v[i].y, mine ? vn.z : T.v[i].z, mine ? vn.w : T.v[i].w);
         }
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
     tile_update(a, L, q, T, j, grp, m, l, acc);
   };
@@ -1674,21 +1737,47 @@ __global__ __launch_bounds__(64 * row_max_waves(kMulti)) void paged_decode_row_k
   // Wave 0: lane -> (head h = lane / 32, dims 4*(lane%32)..+4), merging the W states.
   const int h = lane >> 5;
   const int d0 = (lane & 31) * 4;
+  // Each group's LDS reads are all in flight before the first is used, those of absent waves (inside the array, never
+  // used) among them; a loop over the W states waited for two LDS latencies each.
+  constexpr int kU = kBal ? kBalWaves : 8;
   float M = kMaxSeed;
-  for (int v = 0; v < W; ++v) M = fmaxf(M, rec[v][kG * kD + h]);
+#pragma unroll
+  for (int v0 = 0; v0 < kWaves; v0 += kU) {
+    if (v0 >= W) break;
+    float mv[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) mv[u] = rec[v0 + u][kG * kD + h];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) M = v0 + u < W ? fmaxf(M, mv[u]) : M;
+  }
   float Ls = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int v = 0; v < W; ++v) {
-    const float wgt = fast_exp2(rec[v][kG * kD + h] - M);
-    Ls += rec[v][kG * kD + kG + h] * wgt;
-    const uint4 x = ld16(&rec[v][h * kD + d0]);
-    o[0] += __uint_as_float(x.x) * wgt;
-    o[1] += __uint_as_float(x.y) * wgt;
-    o[2] += __uint_as_float(x.z) * wgt;
-    o[3] += __uint_as_float(x.w) * wgt;
+#pragma unroll
+  for (int v0 = 0; v0 < kWaves; v0 += kU) {
+    if (v0 >= W) break;
+    float mv[kU], lv[kU];
+    uint4 x[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const float* r = rec[v0 + u];
+      mv[u] = r[kG * kD + h];
+      lv[u] = r[kG * kD + kG + h];
+      x[u] = ld16(r + h * kD + d0);
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      if (v0 + u < W) {
+        const float wgt = fast_exp2(mv[u] - M);
+        Ls += lv[u] * wgt;
+        o[0] += __uint_as_float(x[u].x) * wgt;
+        o[1] += __uint_as_float(x[u].y) * wgt;
+        o[2] += __uint_as_float(x[u].z) * wgt;
+        o[3] += __uint_as_float(x[u].w) * wgt;
+      }
+    }
   }
   if (nch > 1) {
     // Chunked form, a row spread over several chunks: this chunk's record, [kG][kD] o then m[kG], l[kG] (fp32).
-    float* r = a.ws + (((int64_t)b * gridDim.z + blockIdx.z) * a.hkv + g) * kRowRec;
+    float* r = a.ws + (((int64_t)b * a.max_splits + ch) * a.hkv + g) * kRowRec;
     st16(r + h * kD + d0, make_uint4(__float_as_uint(o[0]), __float_as_uint(o[1]), __float_as_uint(o[2]),
                                      __float_as_uint(o[3])));
     if ((lane & 31) == 0) {
@@ -1708,32 +1797,45 @@ __global__ __launch_bounds__(64 * row_max_waves(kMulti)) void paged_decode_row_k
 // 4*(l%32)..+4.  The records of every chunk of the grid are loaded at once, before the row's context is known (the
 // combine is one memory round trip); those of chunks past the row's end are stale and are never used.  Rows held by
 // one chunk were written by the row kernel.
-template <bool kAppend>
+// The balanced form knows a row's chunks only from all lengths (one round trip): it loads kBalEager records beside
+// them and the rest of a row that has more after.
+constexpr int kBalEager = 4;
+
+template <bool kAppend, bool kBal = false>
 __global__ __launch_bounds__(64) void paged_decode_chunk_combine_kernel(const DecodeArgs a) {
-  const int b = blockIdx.x;
-  const int g = blockIdx.y;
+  const int b = blockIdx.y;
+  const int g = blockIdx.x;
   const int lane = threadIdx.x;
   const int h = lane >> 5;
   const int d0 = (lane & 31) * 4;
-  const int nchg = a.max_splits;  // chunks per row in the grid, <= kChunkMax
+  const int nchg = a.max_splits;  // records per row, <= kChunkMax
   const float* base = a.ws + ((int64_t)b * nchg * a.hkv + g) * kRowRec;
   uint4 o[kChunkMax];
   float mr[kChunkMax], lr[kChunkMax];
-#pragma unroll
-  for (int u = 0; u < kChunkMax; ++u) {
+  auto load = [&](int u, int n) __attribute__((always_inline)) {
     o[u] = make_uint4(0u, 0u, 0u, 0u);
     mr[u] = kMaxSeed;
     lr[u] = 0.f;
-    if (u < nchg) {
+    if (u < n) {
       const float* r = base + (int64_t)u * a.hkv * kRowRec;
       o[u] = ld16(r + h * kD + d0);
       mr[u] = r[kG * kD + h];
       lr[u] = r[kG * kD + kG + h];
     }
+  };
+  constexpr int kEager = kBal ? kBalEager : kChunkMax;
+  const int c_all = kBal ? balanced_seqlens(a, lane) : 0;
+#pragma unroll
+  for (int u = 0; u < kEager; ++u) load(u, nchg);
+  int nch;
+  if constexpr (kBal) {
+    nch = readlane(balanced_split<kAppend>(a, c_all, lane).nch, b);
+  } else {
+    nch = (row_ctx<kAppend>(a, b) + a.split_tokens - 1) / a.split_tokens;
   }
-  const int ctx = row_ctx<kAppend>(a, b);
-  const int nch = (ctx + a.split_tokens - 1) / a.split_tokens;
   if (nch <= 1) return;
+#pragma unroll
+  for (int u = kEager; u < kChunkMax; ++u) load(u, nch);
   float M = kMaxSeed;
 #pragma unroll
   for (int u = 0; u < kChunkMax; ++u)
@@ -1805,6 +1907,19 @@ int sk_grid_of(int hkv, int form) {
   return g;
 }
 
+// Workgroups per KV head of the balanced form the current device holds at once (4 waves a SIMD; cached per device).
+int bal_resident(int hkv) {
+  static std::atomic<int> cache[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256 * 4 / hkv;
+  int cus = cache[dev].load(std::memory_order_relaxed);
+  if (cus <= 0) {
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 256 * 4 / hkv;
+    cache[dev].store(cus, std::memory_order_relaxed);
+  }
+  return cus * 4 / hkv;
+}
+
 int sk_grid(int hkv) {
   const int g0 = sk_grid_of(hkv, 0), g1 = sk_grid_of(hkv, 1), g2 = hkv <= 8 ? sk_grid_of(hkv, 2) : 0;
   return std::max(g0, std::max(g1, g2));
@@ -1818,7 +1933,7 @@ int sk_effective_grid_host(int grid, int64_t nt) {
 
 // The decompositions of one decode call.  split_tokens == 0 lets choose_path pick; Q3A_DECODE_ROW,
 // Q3A_DECODE_CHUNKS and Q3A_DECODE_STREAMK (negative codes) ask for one; split_tokens > 0 is the fixed split.
-enum class Path { kNone, kRow, kChunks, kStreamK, kFixed };
+enum class Path { kNone, kRow, kChunks, kBalanced, kStreamK, kFixed };
 
 // Chunked form geometry for a table of cap_tiles tiles: W waves of `per` tiles per chunk, nch chunks per row.
 // 128-token chunks (8 waves of one tile) while 16 of them cover the table, then 16 waves of one tile, then 8
@@ -1842,6 +1957,34 @@ bool chunk_geometry(int64_t cap_tiles, int* W, int* per, int* nch) {
 // Batches up to which long rows take the chunked form, and the table capacity (tiles) from which they do.
 constexpr int kChunkMaxBatch = 16;
 constexpr int kChunkMinTiles = 2 * kMaxRowTiles;
+
+// The balanced form takes kBalMinBatch..kBalMaxBatch rows (a lane each) of tables up to 2,048 tokens, from 272 tokens
+// (up to 16 rows) or 528 (more rows, at most 8 KV heads).  Norm/rope form, us per call in a graph of 28, against the form
+// that served the shape before:
+//   below 5 rows the chunks are few and the extra round trip shows (chunks / balanced: 1 x 1,000 8.3 / 8.6,
+//     4 x 1,000 10.0 / 10.1); 5 to 16 rows: 16 x U[300, 1020] 18.7 / 14.9, 8 x U[900, 1780] 19.0 / 15.5, 8 x 500 9.9 / 9.9
+//   two tiles a wave (tables of 256 tokens) are one launch of the row kernel: 8 x U[50, 250] 8.4 in chunks, 7.8
+//   17 to 64 rows (row kernel / balanced): 24 rows log-uniform in [178, 1780] 26.1 / 19.7, 64 46.4 / 38.4, 20 x U[500, 1000]
+//     18.9 / 17.4, 40 x U[890, 1780] 46.1 / 41.4.  Up to 512 tokens the row kernel's single launch wins (24 x 490 13.3 / 15.4),
+//     and up to 1,024 where its workgroups fill the CUs once (25 to 32 rows: 28 x U[500, 1000] 21.8 / 22.7, log-uniform in
+//     [100, 1000] 18.5 / 17.0).  Rows of nearly one length (within 5 %) lose the combine launch: 24 x 975 21.6 / 23.3,
+//     28 x 1,735 38.7 / 40.8, 64 x 1,735 74.5 / 78.6; the host does not know the lengths, and ragged rows are the rule.
+constexpr int kRowOneTiles = 16;
+constexpr int kBalMinBatch = 5;
+constexpr int kBalMaxBatch = 64;
+
+bool balanced_ok(int batch, int hkv, int64_t max_ctx) {
+  const int64_t cap_tiles = (max_ctx + kTile - 1) / kTile;
+  if (batch < kBalMinBatch || batch > kBalMaxBatch || cap_tiles > kRowMaxWaves * kRowMaxPer) return false;
+  if (batch <= kChunkMaxBatch) return cap_tiles > kRowOneTiles;
+  const int cu_rows = bal_resident(hkv) / 4;  // rows whose workgroups in the row kernel are one per CU
+  const bool fills = batch <= cu_rows && 4 * batch > 3 * cu_rows;
+  return hkv <= 8 && cap_tiles > (fills ? 4 : 2) * kRowOneTiles;
+}
+
+// Its shortest chunk (tiles): two tiles a wave, so a 2,048-token row has at most kChunkMax records and up to 16 rows
+// need no more workspace than their 128-token chunks; more rows than 32 fill the device with twice that.
+int bal_min_tiles(int batch) { return batch <= 32 ? 8 : 16; }
 
 Path choose_path(int batch, int64_t max_ctx, int split_tokens) {
   const int64_t cap_tiles = (max_ctx + kTile - 1) / kTile;
@@ -1867,8 +2010,14 @@ Path choose_path(int batch, int64_t max_ctx, int split_tokens) {
 
 size_t workspace_bytes(int batch, int hkv, int max_pages, int page_size, int split_tokens) {
   const int64_t max_ctx = (int64_t)max_pages * page_size;
+  if (split_tokens == Q3A_WORKSPACE_BALANCED) {
+    if (balanced_ok(batch, hkv, max_ctx))
+      return (size_t)batch * ceil_div(ceil_div(max_ctx, kTile), bal_min_tiles(batch)) * hkv * kRowRec * sizeof(float);
+    split_tokens = 0;
+  }
   switch (choose_path(batch, max_ctx, split_tokens)) {
     case Path::kNone:
+    case Path::kBalanced:  // never choose_path's
     case Path::kRow: return 0;
     case Path::kChunks: {
       int w, p, n;
@@ -2088,8 +2237,19 @@ static int launch_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
                 (long long)page_extent);
   const int64_t max_ctx = (int64_t)max_pages_per_seq * page_size;
   if (max_ctx > (int64_t)1 << 30) return fail(Q3A_EINVAL, "%s: context capacity too large", who);
-  const int workspace_split = split_tokens;  // the value the caller sized the workspace with
-  const Path path = choose_path(batch, max_ctx, split_tokens);
+  Path path = choose_path(batch, max_ctx, split_tokens);
+  const bool bal_fits = balanced_ok(batch, num_kv_heads, max_ctx);
+  if (split_tokens == 0) {
+    // The balanced form where the workspace holds its records; a table of two tiles a wave takes the row kernel
+    // whatever the batch (the workspace stays that of the chunks).
+    if (bal_fits && workspace != nullptr && (uintptr_t)workspace % 16 == 0 &&
+        workspace_bytes_ >= workspace_bytes(batch, num_kv_heads, max_pages_per_seq, page_size, Q3A_WORKSPACE_BALANCED))
+      path = Path::kBalanced;
+    else if (path == Path::kChunks && max_ctx <= kRowOneTiles * kTile)
+      path = Path::kRow;
+  }
+  // The value the caller sized the workspace with.
+  const int workspace_split = path == Path::kBalanced ? Q3A_WORKSPACE_BALANCED : split_tokens;
   if (path == Path::kNone)
     return fail(Q3A_EINVAL, "%s: decode path %d does not take this shape (batch %d, table of %lld tokens)", who,
                 split_tokens, batch, (long long)max_ctx);
@@ -2099,11 +2259,13 @@ static int launch_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
   // chunks of the row, so the row's tiles spread over many CUs, and a combine.
   const bool row = path == Path::kRow;
   const bool chunks = path == Path::kChunks;
+  const bool bal = path == Path::kBalanced;
   const int cap_tiles = (int)((max_ctx + kTile - 1) / kTile);
-  int row_waves = std::min(cap_tiles, row_max_waves(cap_tiles > kRowMaxWaves)), chunk_per = 1, nchunks = 1;
+  int row_waves = std::min(cap_tiles, kRowMaxWaves / 2), chunk_per = 1, nchunks = 1;
   if (chunks) chunk_geometry(cap_tiles, &row_waves, &chunk_per, &nchunks);
   if (row) split_tokens = cap_tiles * kTile;
   if (chunks) split_tokens = row_waves * chunk_per * kTile;
+  if (bal) split_tokens = bal_min_tiles(batch) * kTile;
   const bool sk = path == Path::kStreamK;
   if (sk) split_tokens = 0;
   if (path == Path::kFixed && split_tokens == 0)
@@ -2138,7 +2300,7 @@ static int launch_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
   }
   if (nr != nullptr) {
     if (!append) return fail(Q3A_EINVAL, "%s: the norm/rope form needs k_new/v_new", who);
-    if (!row && !sk && !chunks)
+    if (!row && !sk && !chunks && !bal)
       return fail(Q3A_EINVAL, "%s: the norm/rope form needs split_tokens <= 0 and batch <= %d", who, kSkMaxRows);
     if (sk && num_kv_heads > 8)
       return fail(Q3A_EINVAL, "%s: the norm/rope form supports at most 8 KV heads (got %d)", who, num_kv_heads);
@@ -2272,33 +2434,79 @@ static int launch_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
   a.grid = 0;
   a.prefix = nullptr;
   a.ws = static_cast<float*>(workspace);
+  if (bal) {
+    // a.grid: chunks per KV head to aim for, short of the resident workgroups by half the batch (a row's chunks are
+    // rounded up).  More than 32 rows have one or two chunks each there, too coarse to even the CUs out: they aim for
+    // twice as many (64 x U[500, 1000] 41.7 -> 39.8 us per call, 64 x U[890, 1780] 67.3 -> 62.9; up to 32 rows 24.2 -> 26.1
+    // the other way).  The chunk length is at least total / a.grid, so the chunks number at most a.grid + batch.
+    a.row_per = bal_min_tiles(batch);
+    a.grid = std::max(1, (batch > 32 ? 2 : 1) * bal_resident(num_kv_heads) - batch / 2);
+    const dim3 bgrid(num_kv_heads, std::min(a.grid + batch, batch * max_splits)), bblock(64 * kBalWaves);
+    if (rope)
+      hipLaunchKernelGGL((paged_decode_row_kernel<true, true, true, true>), bgrid, bblock, 0, st, a);
+    else if (append)
+      hipLaunchKernelGGL((paged_decode_row_kernel<true, true, false, true>), bgrid, bblock, 0, st, a);
+    else
+      hipLaunchKernelGGL((paged_decode_row_kernel<false, true, false, true>), bgrid, bblock, 0, st, a);
+    e = hipGetLastError();
+    if (e != hipSuccess) return fail(Q3A_ELAUNCH, "%s: balanced launch failed: %s", who, hipGetErrorString(e));
+    const dim3 cgrid(num_kv_heads, batch);
+    if (append)
+      hipLaunchKernelGGL((paged_decode_chunk_combine_kernel<true, true>), cgrid, dim3(64), 0, st, a);
+    else
+      hipLaunchKernelGGL((paged_decode_chunk_combine_kernel<false, true>), cgrid, dim3(64), 0, st, a);
+    e = hipGetLastError();
+    if (e != hipSuccess) return fail(Q3A_ELAUNCH, "%s: combine launch failed: %s", who, hipGetErrorString(e));
+    return Q3A_OK;
+  }
   if (row || chunks) {
     a.row_per = chunks ? chunk_per : (cap_tiles + row_waves - 1) / row_waves;
-    const dim3 rgrid(batch, num_kv_heads, chunks ? nchunks : 1), rblock(64 * row_waves);
-    if (a.row_per == 1) {
-      if (rope)
-        hipLaunchKernelGGL((paged_decode_row_kernel<true, false, true>), rgrid, rblock, 0, st, a);
-      else if (append)
-        hipLaunchKernelGGL((paged_decode_row_kernel<true, false>), rgrid, rblock, 0, st, a);
-      else
-        hipLaunchKernelGGL((paged_decode_row_kernel<false, false>), rgrid, rblock, 0, st, a);
-    } else {
-      if (rope)
-        hipLaunchKernelGGL((paged_decode_row_kernel<true, true, true>), rgrid, rblock, 0, st, a);
-      else if (append)
-        hipLaunchKernelGGL((paged_decode_row_kernel<true, true>), rgrid, rblock, 0, st, a);
-      else
-        hipLaunchKernelGGL((paged_decode_row_kernel<false, true>), rgrid, rblock, 0, st, a);
-    }
-    e = hipGetLastError();
-    if (e != hipSuccess) return fail(Q3A_ELAUNCH, "%s: row launch failed: %s", who, hipGetErrorString(e));
-    if (chunks && nchunks > 1) {
-      if (append)
-        hipLaunchKernelGGL(paged_decode_chunk_combine_kernel<true>, dim3(batch, num_kv_heads), dim3(64), 0, st, a);
-      else
-        hipLaunchKernelGGL(paged_decode_chunk_combine_kernel<false>, dim3(batch, num_kv_heads), dim3(64), 0, st, a);
+    // The row is grid dimension y, which holds 65,535: larger batches go in slices of rows.
+    constexpr int kGridRows = 65535;
+    for (int row0 = 0; row0 < batch; row0 += kGridRows) {
+      const int rows = std::min(batch - row0, kGridRows);
+      if (row0 > 0) {
+        a.q += kGridRows * a.q_sb;
+        a.seqlens += kGridRows;
+        a.bt += kGridRows * a.bt_sb;
+        a.out += kGridRows * a.o_sb;
+        if (append) {
+          a.k_new += kGridRows * a.kn_sb;
+          a.v_new += kGridRows * a.vn_sb;
+        }
+        if (rope) {
+          a.rcos += kGridRows * a.rs_sb;
+          a.rsin += kGridRows * a.rs_sb;
+        }
+        if (chunks && nchunks > 1) a.ws += (int64_t)kGridRows * nchunks * num_kv_heads * kRowRec;
+      }
+      const dim3 rgrid(num_kv_heads, rows, chunks ? nchunks : 1), rblock(64 * row_waves);
+      if (a.row_per == 1) {
+        if (rope)
+          hipLaunchKernelGGL((paged_decode_row_kernel<true, false, true>), rgrid, rblock, 0, st, a);
+        else if (append)
+          hipLaunchKernelGGL((paged_decode_row_kernel<true, false>), rgrid, rblock, 0, st, a);
+        else
+          hipLaunchKernelGGL((paged_decode_row_kernel<false, false>), rgrid, rblock, 0, st, a);
+      } else {
+        if (rope)
+          hipLaunchKernelGGL((paged_decode_row_kernel<true, true, true>), rgrid, rblock, 0, st, a);
+        else if (append)
+          hipLaunchKernelGGL((paged_decode_row_kernel<true, true>), rgrid, rblock, 0, st, a);
+        else
+          hipLaunchKernelGGL((paged_decode_row_kernel<false, true>), rgrid, rblock, 0, st, a);
+      }
       e = hipGetLastError();
-      if (e != hipSuccess) return fail(Q3A_ELAUNCH, "%s: chunk combine launch failed: %s", who, hipGetErrorString(e));
+      if (e != hipSuccess) return fail(Q3A_ELAUNCH, "%s: row launch failed: %s", who, hipGetErrorString(e));
+      if (chunks && nchunks > 1) {
+        const dim3 cgrid(num_kv_heads, rows);
+        if (append)
+          hipLaunchKernelGGL(paged_decode_chunk_combine_kernel<true>, cgrid, dim3(64), 0, st, a);
+        else
+          hipLaunchKernelGGL(paged_decode_chunk_combine_kernel<false>, cgrid, dim3(64), 0, st, a);
+        e = hipGetLastError();
+        if (e != hipSuccess) return fail(Q3A_ELAUNCH, "%s: chunk combine launch failed: %s", who, hipGetErrorString(e));
+      }
     }
     return Q3A_OK;
   }

@@ -1,0 +1,132 @@
+"""GPU parity of the balanced decode (the library's own choice for 5 to 64 rows): chunks cut on the
+device from all rows' lengths.
+
+* against the oracle (bf16 output within max-abs 2e-2 and mean-abs 2e-3 of the fp32-softmax restatement of
+  engine/talker.py:82-88) at the edges of its range: the smallest and largest batch and table, one lane short of a wave,
+  rows of 0, 1, a tile, a tile and a token, and full tables, all rows full (the longest chunks) and all rows empty but one;
+* the plain form bit-identical to the append form on the same tokens, and that with the norm/rope form on +-1 rows,
+  whose normalised rows are exact (the same decomposition in all three);
+* the shapes just outside its range, against the oracle; a call whose workspace does not hold its records is the row
+  kernel's.
+"""
+import numpy as np
+import pytest
+import torch
+
+import q3attn
+from helpers import decode_oracle, to_np
+from oracle import attention as ora
+from q3attn import _lib
+from q3attn import workloads as W
+
+
+def _ctx(B, cap, kind):
+    rng = np.random.default_rng(B * 7 + cap)
+    if kind == "full":
+        return np.full(B, cap)
+    if kind == "lone":
+        c = np.zeros(B, np.int64)
+        c[B // 2] = cap
+        return c
+    c = np.rint(np.exp(rng.uniform(0, np.log(cap), size=B))).astype(np.int64)
+    c[:5] = [0, 1, 16, 17, cap]
+    return rng.permutation(c)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["ragged", "full", "lone"])
+@pytest.mark.parametrize("B,cap", [(5, 272), (5, 2048), (16, 1040), (17, 528), (32, 1040), (33, 544), (63, 1024), (64, 2048)])
+def test_balanced_vs_oracle_and_append(cuda_device, B, cap, kind):
+    ctx = _ctx(B, cap, kind)
+    wl = W.make_decode("bal", cuda_device, ctx=ctx, num_pages=2 * B * (cap // 16 + 1), max_ctx=cap, seed=B + cap)
+    L = wl.layers[0]
+    out = q3attn.paged_decode(L.q, wl.k_cache, wl.v_cache, wl.cache_seqlens, L.block_table, wl.scale)
+    ok, st = ora.compare(to_np(out), decode_oracle(wl))
+    assert ok, (B, cap, kind, st)
+    assert not out[torch.from_numpy(ctx == 0).to(cuda_device)].float().abs().sum().item()
+    # The append form, its slots poisoned: same bits, and the pool as index_copy_ leaves it.
+    page = wl.page_size
+    bt = L.block_table.cpu().numpy().astype(np.int64)
+    live = ctx > 0
+    pos = np.maximum(ctx - 1, 0)
+    slots = torch.from_numpy((bt[np.arange(B), pos // page] * page + pos % page)[live]).to(cuda_device)
+    rows = torch.from_numpy(np.flatnonzero(live)).to(cuda_device)
+    kf, vf = (x.view(-1, W.HKV, W.HEAD_DIM) for x in (wl.k_cache, wl.v_cache))
+    k, v = torch.zeros((2, B, W.HKV, W.HEAD_DIM), dtype=torch.bfloat16, device=cuda_device)
+    k[rows], v[rows] = kf[slots], vf[slots]
+    ref_k, ref_v = wl.k_cache.clone(), wl.v_cache.clone()
+    kf[slots], vf[slots] = float("nan"), float("nan")
+    old = torch.from_numpy(ctx - 1).to(torch.int32).to(cuda_device)
+    app = q3attn.paged_decode_append(L.q, k, v, wl.k_cache, wl.v_cache, old, L.block_table, wl.scale)
+    assert torch.equal(app, out)
+    assert torch.equal(wl.k_cache, ref_k) and torch.equal(wl.v_cache, ref_v)
+
+
+@pytest.mark.gpu
+def test_balanced_rope_form_exact_rows(cuda_device):
+    dev = cuda_device
+    ctx = _ctx(20, 1024, "ragged")
+    wl = W.make_decode("bal_rope", dev, ctx=ctx, num_pages=4096, max_ctx=1024, seed=7)
+    rng = np.random.default_rng(5)
+    r = lambda x: ora.bf16_round(np.asarray(x, np.float32))
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x, np.float32)).to(dev).to(torch.bfloat16)
+    q, k = (r(rng.choice([-1.0, 1.0], size=(20, h, W.HEAD_DIM))) for h in (W.HQ, W.HKV))
+    v = r(rng.standard_normal((20, W.HKV, W.HEAD_DIM)))
+    qn, kn = (r(rng.uniform(0.5, 1.5, W.HEAD_DIM)) for _ in range(2))
+    cos_t, sin_t = ora.rope_tables(1024)
+    pos = np.maximum(ctx - 1, 0)
+    cos, sin = r(cos_t[pos]), r(sin_t[pos])
+    qq, kk = (ora.norm_rope(x, w, cos[:, None], sin[:, None], 0.0, eager=False) for x, w in ((q, qn), (k, kn)))
+    old = torch.from_numpy(ctx - 1).to(torch.int32).to(dev)
+    L = wl.layers[0]
+    kc, vc = wl.k_cache.clone(), wl.v_cache.clone()
+    out = q3attn.paged_decode_append_rope(t(q), t(k), t(v), t(qn), t(kn), t(cos), t(sin), wl.k_cache, wl.v_cache, old,
+                                          L.block_table, wl.scale, 0.0)
+    ref = q3attn.paged_decode_append(t(qq), t(kk), t(v), kc, vc, old, L.block_table, wl.scale)
+    assert torch.equal(out, ref) and torch.equal(kc, wl.k_cache) and torch.equal(vc, wl.v_cache)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,cap", [(4, 1024), (65, 1024), (8, 256), (17, 512), (28, 1024), (8, 2064)])
+def test_shapes_beside_its_range(cuda_device, B, cap):
+    wl = W.make_decode("bal_no", cuda_device, ctx=_ctx(max(B, 5), cap, "ragged")[:B], num_pages=4 * B * 130, max_ctx=cap, seed=B)
+    L = wl.layers[0]
+    out = q3attn.paged_decode(L.q, wl.k_cache, wl.v_cache, wl.cache_seqlens, L.block_table, wl.scale)
+    ok, st = ora.compare(to_np(out), decode_oracle(wl))
+    assert ok, st
+
+
+@pytest.mark.gpu
+def test_without_the_workspace_the_row_kernel(cuda_device):
+    """17 to 64 rows need no workspace (q3a_paged_decode_workspace_bytes of split_tokens 0 is 0): without one the call is
+    the row kernel's, bit for bit."""
+    wl = W.make_decode("bal_ws", cuda_device, ctx=_ctx(20, 1024, "ragged"), num_pages=4096, max_ctx=1024, seed=3)
+    L, lib = wl.layers[0], _lib.lib()
+    out = torch.empty_like(L.q)
+    rc = lib.q3a_paged_decode(L.q.data_ptr(), L.q.stride(0), L.q.stride(1), wl.k_cache.data_ptr(), wl.v_cache.data_ptr(),
+                              *wl.k_cache.stride()[:3], wl.k_cache.shape[0], wl.page_size, wl.cache_seqlens.data_ptr(),
+                              L.block_table.data_ptr(), L.block_table.stride(0), L.block_table.shape[1], out.data_ptr(),
+                              out.stride(0), out.stride(1), None, 0, 20, W.HQ, W.HKV, W.HEAD_DIM, wl.scale, 0,
+                              torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    row = q3attn.paged_decode(L.q, wl.k_cache, wl.v_cache, wl.cache_seqlens, L.block_table, wl.scale, q3attn.DECODE_ROW)
+    assert torch.equal(out, row)
+
+
+def test_workspace_query():
+    """The balanced form's records, 8 tiles a chunk (16 above 32 rows); elsewhere the bytes of split_tokens 0."""
+    ws = lambda B, pages, split, hkv=8: _lib.lib().q3a_paged_decode_workspace_bytes(B, 2 * hkv, hkv, 128, pages, 16, split)
+    assert ws(16, 128, -5) == ws(16, 128, 0) == 16 * 16 * 8 * 1040
+    assert ws(20, 65, -5) == 20 * 9 * 8 * 1040 and ws(64, 128, -5) == 64 * 8 * 8 * 1040
+    for B, pages, hkv in ((4, 128, 8), (65, 128, 8), (8, 16, 8), (17, 32, 8), (28, 64, 8), (8, 129, 8), (20, 65, 16)):
+        assert ws(B, pages, -5, hkv) == ws(B, pages, 0, hkv)
+
+
+def test_chunk_count_arithmetic():
+    """ceil(n / d) as the kernel forms it, (n + d - 1/2) * rcp(d) truncated, with rcp off by one step either way."""
+    d = np.arange(1, 8193, dtype=np.int64)[:, None]
+    rcp = (np.float32(1) / d.astype(np.float32)).astype(np.float32)
+    for n in range(0, 8193, 61):
+        x = np.float32(n) + d.astype(np.float32) - np.float32(0.5)
+        for r in (rcp, np.nextafter(rcp, np.float32(0)), np.nextafter(rcp, np.float32(2))):
+            assert np.array_equal((x * r).astype(np.int64), -(-n // d)), n
