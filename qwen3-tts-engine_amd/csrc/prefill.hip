@@ -35,7 +35,7 @@ namespace {
 
 constexpr int kD = 128;
 constexpr int kG = 2;  // query heads per KV head (the softmax below is written for exactly two)
-constexpr int kQT = 64;        // query tokens per workgroup (16 per wave, both heads)
+constexpr int kQT64 = 64;      // query tokens per workgroup of the unsplit kernel (16 per wave, both heads)
 constexpr int kKT = 32;        // keys per LDS tile
 constexpr int kRowB = kD * 2;  // bytes of one key row in an LDS tile
 constexpr int kTileB = kKT * kRowB;
@@ -117,14 +117,23 @@ __device__ __forceinline__ uint2 ldtr(const uint8_t* lds) {
 __device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 // Three waves per SIMD (<= 168 VGPRs): three workgroups per CU hide each other's prologues and barriers.
-template <bool kGrouped, bool kRopeQ = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void prefill_kernel(const PrefillArgs a) {
+//
+// Key-split form (kS > 1), for calls whose grid leaves CUs idle: kS teams of kQW waves share a workgroup's 16 kQW query
+// tokens, team i taking key tiles i, i + kS, ... through stages of its own; the teams' (m, l, O) merge in LDS at the
+// end.  The call is then bound by the prologue and a kS-th of the key-tile chain instead of the whole chain on one wave
+// per SIMD.
+template <bool kGrouped, bool kRopeQ = false, int kQW = 4, int kS = 1>
+__global__ __launch_bounds__(64 * kQW * kS) __attribute__((amdgpu_waves_per_eu(kS == 1 ? 3 : 2, kS == 1 ? 3 : 2)))
+void prefill_kernel(const PrefillArgs a) {
+  static_assert(kQW == 2 || kQW == 4, "a team's waves divide the 4 groups of a K/V tile");
+  static_assert(kS == 1 || !kGrouped, "the grouped order is for large grids");
+  constexpr int kQT = 16 * kQW;  // query tokens per workgroup (16 per wave, both heads)
   // Two stages of K and V tiles; separate arrays so the compiler can tell the stage being filled from the one
   // being read.
-  __shared__ __align__(16) uint8_t sK0[kTileB];
-  __shared__ __align__(16) uint8_t sV0[kTileB];
-  __shared__ __align__(16) uint8_t sK1[kTileB];
-  __shared__ __align__(16) uint8_t sV1[kTileB];
+  __shared__ __align__(16) uint8_t sK0[kS * kTileB];
+  __shared__ __align__(16) uint8_t sV0[kS * kTileB];
+  __shared__ __align__(16) uint8_t sK1[kS * kTileB];
+  __shared__ __align__(16) uint8_t sV1[kS * kTileB];
 
   // Grid x = (sequence, KV head) with the head fastest, z = query tile reversed (slowest): the tiles with the
   // most key tiles (the last ones of each sequence) dispatch first, the short ones fill in last.  Workgroups
@@ -149,17 +158,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     if (s >= a.nseq) return;
   }
   const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_wg = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = kS == 1 ? wave_wg : wave_wg & (kQW - 1);  // of the team
+  const int team = kS == 1 ? 0 : wave_wg / kQW;
   const int lane = tid & 63;
   const int col = lane & 15;
   const int g4 = lane >> 4;
 
   // The sequence's first 64 page ids depend only on s: fetch them before cu_seqlens so the first tile's
   // loads wait for one memory round trip, not two.
-  // Waves 0 and 1 copy K tiles, waves 2 and 3 V tiles (below); each uses its operand's own strides, which are
+  // A team's first half copies K tiles, the second V tiles (below); each uses its operand's own strides, which are
   // wave-uniform and stay in scalar registers.  The norm/rope-q form reads K paged (the pool, where its producer
   // pass stored the normalised rows) and V packed.
-  const bool copies_k = wave < 2;
+  const bool copies_k = wave < kQW / 2;
   const bool paged = a.bt != nullptr && (!kRopeQ || copies_k);
   const int64_t bt_row = (int64_t)s * a.bt_sb;
   const int64_t c_sp = copies_k ? a.k_sp : a.v_sp;
@@ -178,7 +189,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   int page0 = -1;
   if (paged) {
     typedef __attribute__((address_space(4))) const int32_t cint32;
-    const int pi0 = (16 * (wave & 1)) >> a.page_shift;
+    const int pi0 = (kKT * team + 16 * (wave & (kQW / 2 - 1))) >> a.page_shift;
     if (pi0 < a.max_pages) page0 = ((const cint32*)a.bt)[bt_row + pi0];
   }
 
@@ -302,14 +313,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
       }
     }
   };
-  if (!kRopeQ && a.pk != nullptr && !pool_from_lds) load_rows(chunked ? a.p_first + qt * kQT : kown0);
+  if (!kRopeQ && a.pk != nullptr && !pool_from_lds && team == 0) load_rows(chunked ? a.p_first + qt * kQT : kown0);
 
   int kend = Lk;
   if (a.causal) {
     const int last = min(Lq - 1, qt * kQT + kQT - 1);
     kend = min(Lk, Lk - Lq + last + 1);
   }
-  const int ntiles = kend > 0 ? (kend + kKT - 1) / kKT : 0;
+  const int ntiles_all = kend > 0 ? (kend + kKT - 1) / kKT : 0;
+  const int ntiles = (ntiles_all - team + kS - 1) / kS;   // of this team: key tiles team, team + kS, ...
+  const int nrounds = (ntiles_all + kS - 1) / kS;         // team 0's, the most
   const int jlim = a.causal ? min(Lk - 1, qpos) : Lk - 1;  // last key this lane's token sees
   // Last key that every token of this wave sees (wave-uniform).
   const int wlim = a.causal ? min(Lk - 1, Lk - Lq + qt * kQT + wave * 16) : Lk - 1;
@@ -326,10 +339,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   // zeros.  Lane l of instruction i lands at LDS chunk slot l & 15 of row rr = 4i + (l >> 4), so it fetches
   // global chunk (l & 15) ^ rr: the swizzle is applied on the global side.  Page ids come from a lane-wise
   // window (lane i = table entry pwin_base + i), read with v_readlane; it is refilled once per 64 pages.
-  static_assert(kKT == 32 && kQT == 64, "the copy assignment below is for 4 waves and 2 groups per tile");
-  const int cgrp = wave & 1;                     // the 16-key group of a tile this wave copies
+  static_assert(kKT == 32, "the copy assignment below is for 2 groups per tile");
+  constexpr int kGroupsPerWave = 4 / kQW;
+  const int cgrp0 = wave & (kQW / 2 - 1);        // the 16-key group(s) of a tile this wave copies
   const uint16_t* cbase = copies_k ? a.k : a.v;  // waves 0, 1 copy K; waves 2, 3 copy V
-  auto group_rsrc = [&](const uint16_t* base, int t, int page) __attribute__((always_inline)) {
+  auto group_rsrc = [&](const uint16_t* base, int t, int cgrp, int page) __attribute__((always_inline)) {
     const int j0 = t * kKT + 16 * cgrp;
     const int nv = min(16, Lk - j0);
     bool ok = nv > 0;
@@ -348,20 +362,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     const int rr = 4 * i + (lane >> 4);
     dma_off[i] = (uint32_t)((rr * c_st + 8 * ((lane & 15) ^ rr)) * 2);
   }
-  // Tile 0 (first = true) takes its page id from the scalar load above.
-  auto issue = [&](int t, uint8_t* Kst, uint8_t* Vst, bool first = false) __attribute__((always_inline)) {
-    int page = 0;
-    if (paged && first) {
-      page = page0;
-    } else if (paged) {
-      const int pi = (t * kKT + 16 * cgrp) >> a.page_shift;
-      if (pi < pwin_base || pi >= pwin_base + 64) load_window(pi & ~63);
-      page = readlane(pwin, pi - pwin_base);
-    }
-    const __amdgpu_buffer_rsrc_t rc = group_rsrc(cbase, t, page);
-    uint8_t* dst = copies_k ? Kst : Vst;
+  // i: the team's i-th tile.  Tile 0 (first = true) takes its first group's page id from the scalar load above.
+  auto issue = [&](int i, uint8_t* Kst, uint8_t* Vst, bool first = false) __attribute__((always_inline)) {
+    const int t = team + kS * i;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dma16(rc, dst + (16 * cgrp + 4 * i) * kRowB, dma_off[i]);
+    for (int c = 0; c < kGroupsPerWave; ++c) {
+      const int cgrp = cgrp0 + c;
+      int page = 0;
+      if (paged && first && c == 0) {
+        page = page0;
+      } else if (paged) {
+        const int pi = (t * kKT + 16 * cgrp) >> a.page_shift;
+        if (pi < pwin_base || pi >= pwin_base + 64) load_window(pi & ~63);
+        page = readlane(pwin, pi - pwin_base);
+      }
+      const __amdgpu_buffer_rsrc_t rc = group_rsrc(cbase, t, cgrp, page);
+      uint8_t* dst = (copies_k ? Kst : Vst) + team * kTileB;
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) dma16(rc, dst + (16 * cgrp + 4 * i4) * kRowB, dma_off[i4]);
+    }
   };
 
   // Operand read offsets.  K (A of S^T): lane (col, g4) reads key kb*16 + col, logical chunk 4kk + g4, stored at
@@ -382,8 +401,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     for (int db = 0; db < 8; ++db) acc[hh][db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m[kG] = {kMaxSeed, kMaxSeed}, l[kG] = {0.f, 0.f};
 
-  auto compute = [&](int t, const uint8_t* Ks, const uint8_t* Vs) __attribute__((always_inline)) {
+  auto compute = [&](int i, const uint8_t* Kst, const uint8_t* Vst) __attribute__((always_inline)) {
+    const int t = team + kS * i;
     if (t * kKT > wmax) return;
+    const uint8_t* Ks = Kst + team * kTileB;
+    const uint8_t* Vs = Vst + team * kTileB;
     // S^T for the tile's 2 blocks of 16 keys, both heads; each K operand is read once.
     f32x4_t st[kG][kKT / 16];
 #pragma unroll
@@ -542,7 +564,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
     __builtin_amdgcn_sched_barrier(0);
   }
-  if (!kRopeQ && a.pk != nullptr && !pool_from_lds) {
+  if (!kRopeQ && a.pk != nullptr && !pool_from_lds && team == 0) {
     store_rows();
     if (chunked) {
       for (int c = qt + nqt_seq; a.p_first + c * kQT < Lk; c += nqt_seq) {
@@ -551,14 +573,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
       }
     }
   }
-  for (int t = 0; t < ntiles; t += 2) {
+  // (Every team runs nrounds rounds, so that all meet every barrier; a team past its last tile computes nothing.)
+  for (int t = 0; t < nrounds; t += 2) {
     if (t + 1 < ntiles) issue(t + 1, sK1, sV1);
-    compute(t, sK0, sV0);
+    if (kS == 1 || t < ntiles) compute(t, sK0, sV0);
     wait_vmem();
     __syncthreads();
-    if (t + 1 >= ntiles) break;
+    if (t + 1 >= nrounds) break;
     if (t + 2 < ntiles) issue(t + 2, sK0, sV0);
-    compute(t + 1, sK1, sV1);
+    if (kS == 1 || t + 1 < ntiles) compute(t + 1, sK1, sV1);
     wait_vmem();
     __syncthreads();
   }
@@ -570,9 +593,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     const int kown1 = min(Lk, kown0 + kQT);
     const int pi0 = kown0 >> a.p_shift;
     constexpr int kParts = kRopeQ ? 1 : 2;
+    constexpr int kThreads = 64 * kQW * kS;
+    static_assert(kQT * 16 % kThreads == 0, "whole passes over a part's chunks");
 #pragma unroll
-    for (int it = 0; it < 4 * kParts; ++it) {
-      const int idx = tid + 256 * it;
+    for (int it = 0; it < kQT * 16 * kParts / kThreads; ++it) {
+      const int idx = tid + kThreads * it;
       const int tl = idx >> (3 + kParts);
       const int part = kRopeQ ? 1 : (idx >> 4) & 1;
       const int ch = idx & 15;
@@ -582,8 +607,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
       if (key < kown1 && pi < a.p_max_pages && (unsigned)page < (unsigned)a.p_pages) {
         const int t = key >> 5;
         const int row = key & (kKT - 1);
-        const uint8_t* stg = part == 0 ? ((t & 1) ? sK1 : sK0) : ((t & 1) ? sV1 : sV0);
-        const uint4 x = ld16(stg + row * kRowB + ((ch ^ (row & 15)) << 4));
+        const bool odd = (t / kS) & 1;  // tile t: stage (t / kS) & 1 of team t mod kS
+        const uint8_t* stg = part == 0 ? (odd ? sK1 : sK0) : (odd ? sV1 : sV0);
+        const uint4 x = ld16(stg + (t % kS) * kTileB + row * kRowB + ((ch ^ (row & 15)) << 4));
         uint16_t* dst = (part == 0 ? a.pk : a.pv) + (int64_t)page * a.p_sp +
                         (int64_t)(key & ((1 << a.p_shift) - 1)) * a.p_st + (int64_t)g * a.p_sh + 8 * ch;
         st16(dst, x);
@@ -599,7 +625,64 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   // of the tile arrays, free once every wave has passed the loop's last barrier (the pool stores above still read
   // them, hence the barrier in that form).  16 B chunks are XOR-swizzled by token, so neither side conflicts.
   if (pool_from_lds) __syncthreads();
-  uint8_t* const so = wave == 0 ? sK0 : (wave == 1 ? sV0 : (wave == 2 ? sK1 : sV1));
+  uint8_t* so;
+  if constexpr (kS == 1) {
+    so = wave == 0 ? sK0 : (wave == 1 ? sV0 : (wave == 2 ? sK1 : sV1));
+  } else {
+    // Teams 1.. hand their state to team 0 through the tile arrays (free as above): slot (team - 1) kQW + wave, 16 KiB
+    // of O (float4 j of lane l at (64 j + l) * 16), kS / 2 slots an array.  A team past the last key tile has l = 0.
+    auto slot_at = [&](int n) __attribute__((always_inline)) {
+      const int arr = n / (kS / 2);
+      return (arr == 0 ? sK0 : (arr == 1 ? sV0 : (arr == 2 ? sK1 : sV1))) + (n % (kS / 2)) * 2 * kTileB;
+    };
+    __shared__ float4 s_ml[kS - 1][kQW][64];
+    if (team > 0) {
+      uint8_t* const d = slot_at((team - 1) * kQW + wave);
+#pragma unroll
+      for (int j = 0; j < 8 * kG; ++j) {
+        const f32x4_t x = acc[j >> 3][j & 7];
+        st16(d + (64 * j + lane) * 16, make_uint4(__float_as_uint(x[0]), __float_as_uint(x[1]), __float_as_uint(x[2]),
+                                                  __float_as_uint(x[3])));
+      }
+      s_ml[team - 1][wave][lane] = make_float4(m[0], m[1], l[0], l[1]);
+    }
+    __syncthreads();
+    if (team > 0) return;
+    float mo[kS - 1][kG], lo[kS - 1][kG], M[kG] = {m[0], m[1]};
+#pragma unroll
+    for (int u = 0; u < kS - 1; ++u) {
+      const float4 x = s_ml[u][wave][lane];
+      mo[u][0] = x.x;
+      mo[u][1] = x.y;
+      lo[u][0] = x.z;
+      lo[u][1] = x.w;
+    }
+#pragma unroll
+    for (int hh = 0; hh < kG; ++hh) {
+#pragma unroll
+      for (int u = 0; u < kS - 1; ++u) M[hh] = fmaxf(M[hh], mo[u][hh]);
+      const float w0 = fast_exp2(m[hh] - M[hh]);
+      l[hh] *= w0;
+#pragma unroll
+      for (int db = 0; db < 8; ++db) acc[hh][db] = acc[hh][db] * w0;
+    }
+#pragma unroll
+    for (int u = 0; u < kS - 1; ++u) {
+      const uint8_t* const d = slot_at(u * kQW + wave);
+#pragma unroll
+      for (int hh = 0; hh < kG; ++hh) {
+        const float wu = fast_exp2(mo[u][hh] - M[hh]);
+        l[hh] += lo[u][hh] * wu;
+#pragma unroll
+        for (int db = 0; db < 8; ++db) {
+          const uint4 x = ld16(d + (64 * (8 * hh + db) + lane) * 16);
+          const f32x4_t o = {__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z), __uint_as_float(x.w)};
+          acc[hh][db] = acc[hh][db] + o * wu;
+        }
+      }
+    }
+    so = slot_at(wave);  // read above by this wave alone
+  }
 #pragma unroll
   for (int hh = 0; hh < kG; ++hh) {
     const float lt = sum_xor32(sum_xor16(l[hh]));
@@ -1186,8 +1269,25 @@ static int resident_slots() {
   return n;
 }
 
+// Teams per workgroup of the key-split form, 0 for the unsplit kernel: where the workgroups leave CUs idle (one per CU
+// at most; its 8 waves of up to 178 registers take a CU) and the key-tile chain is long enough to pay for the merge and
+// the wider prologue, about 1 us.  Four teams of 32 query tokens where they fit, else two of 64.  us per call in a
+// graph, unsplit / split:
+//   packed (the keys are bounded by the longest query range; half of the query tiles see fewer)
+//     1 x 300 8.7 / 9.2, 1 x 400 12.3 / 10.6, 1 x 1,000 24.9 / 16.5, 1 x 2,048 (two teams) 46.2 / 36.4, 2 x 500 15.6 / 12.5
+//   dense (every query tile sees the prefix): 8 x 100 + 50 8.3 / 9.9, 1 x 200 + 100 11.4 / 10.6, 4 x 250 + 150 14.9 / 12.9,
+//     6 x 210 + 170 (two teams) 14.8 / 13.6; two teams below that: 4 x U[150, 400] packed 13.3 / 12.9, 8 x U[150, 250] 18.4 / 19.6
+static int key_split(int num_seqs, int hkv, int max_seqlen_q, bool dense, int seqlen_k) {
+  const int cus = resident_slots() / 3;
+  const int64_t heads = (int64_t)num_seqs * hkv;
+  const int keys = dense ? seqlen_k : max_seqlen_q;
+  if (keys >= (dense ? 288 : 384) && heads * ((max_seqlen_q + 31) / 32) <= cus) return 4;
+  if (keys >= 352 && heads * ((max_seqlen_q + 63) / 64) <= cus) return 2;
+  return 0;
+}
+
 static int launch(const PrefillArgs& args, int num_seqs, int max_seqlen_q, void* stream, const char* who) {
-  const int nqt = (max_seqlen_q + kQT - 1) / kQT;
+  const int nqt = (max_seqlen_q + kQT64 - 1) / kQT64;
   if ((int64_t)num_seqs * args.hkv > 0x7fffffff || nqt > 65535)
     return fail(Q3A_EINVAL, "%s: grid too large (%d seqs x %d KV heads x %d query tiles)", who, num_seqs, args.hkv,
                 nqt);
@@ -1207,7 +1307,19 @@ static int launch(const PrefillArgs& args, int num_seqs, int max_seqlen_q, void*
                        (int64_t)ngroups * nqt <= 65535;
   const dim3 ggrid((1u << a.grp_shift) * a.hkv, 1, ngroups * nqt), grid(num_seqs * a.hkv, 1, nqt);
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (a.qn != nullptr) {
+  const int teams = key_split(num_seqs, args.hkv, max_seqlen_q, args.cu_q == nullptr, args.dense_lk);
+  if (teams != 0) {
+    const int qw = teams == 4 ? 2 : 4;  // waves per team
+    a.nqt = (max_seqlen_q + 16 * qw - 1) / (16 * qw);
+    const dim3 sgrid(num_seqs * a.hkv, 1, a.nqt), sblock(64 * qw * teams);
+    if (teams == 4) {
+      if (a.qn != nullptr) hipLaunchKernelGGL((prefill_kernel<false, true, 2, 4>), sgrid, sblock, 0, st, a);
+      else hipLaunchKernelGGL((prefill_kernel<false, false, 2, 4>), sgrid, sblock, 0, st, a);
+    } else {
+      if (a.qn != nullptr) hipLaunchKernelGGL((prefill_kernel<false, true, 4, 2>), sgrid, sblock, 0, st, a);
+      else hipLaunchKernelGGL((prefill_kernel<false, false, 4, 2>), sgrid, sblock, 0, st, a);
+    }
+  } else if (a.qn != nullptr) {
     if (grouped) hipLaunchKernelGGL((prefill_kernel<true, true>), ggrid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL((prefill_kernel<false, true>), grid, dim3(256), 0, st, a);
   } else {
