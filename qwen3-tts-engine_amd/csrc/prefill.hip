@@ -16,8 +16,10 @@
 // K/V tiles of 32 keys are copied global -> LDS by direct-to-LDS buffer loads (no register staging) into two
 // stages, tile t+1 in flight while tile t is consumed, one barrier per tile.  32-key tiles keep the LDS at 32 KiB
 // and the registers under 168 per lane, so three workgroups share a CU (64-key tiles: two).  LDS tiles are
-// row-major [32 keys][128 dims] with the 16-byte chunks of key k XOR-swizzled by k & 15 (bank-conflict free for both the
-// DMA writes and the operand reads).  v_mfma_f32_16x16x32_bf16 layouts: A lane l = row l%16, k 8*(l/16)..+8;
+// row-major [32 keys][128 dims] with the 16-byte chunks of key k XOR-swizzled, K by k & 15 and V by 2 (k & 7): a K operand
+// read takes one chunk of 16 keys, a V transpose read the same two chunks (32 bytes) of 8 keys, and neither has a bank
+// conflict (V swizzled by k & 15 too, keys 2j and 2j + 1 of a transpose read met in the same banks: a third of the LDS
+// cycles).  v_mfma_f32_16x16x32_bf16 layouts: A lane l = row l%16, k 8*(l/16)..+8;
 // B lane l = column l%16, same k; C lane l = column l%16, rows 4*(l/16)..+4.
 //   S^T = K Q^T  : A = K rows from LDS, B = Q^T (columns = this lane's query token)
 //   O^T = V^T P^T: A = V^T from the row-major V tile through ds_read_b64_tr_b16 (a 16-lane transpose read),
@@ -111,6 +113,12 @@ __device__ __forceinline__ uint2 ldtr(const uint8_t* lds) {
   const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)lds);
   return __builtin_bit_cast(uint2, r);
 }
+
+// Instruction classes of __builtin_amdgcn_sched_group_barrier.
+constexpr int kSchedMfma = 0x008, kSchedDsRead = 0x100;
+
+// The V tiles' swizzle of key row `key`, in 16-byte chunks.
+__device__ __forceinline__ int v_swz(int key) { return (key & 7) << 1; }
 
 // Waits for this wave's outstanding vector-memory operations (the direct-to-LDS copies); vmcnt(0), the other
 // counters untouched.
@@ -337,7 +345,7 @@ void prefill_kernel(const PrefillArgs a) {
   // 1 KiB).  The descriptor covers
   // exactly the group's valid rows of head g: rows past the sequence and groups on an invalid page arrive as
   // zeros.  Lane l of instruction i lands at LDS chunk slot l & 15 of row rr = 4i + (l >> 4), so it fetches
-  // global chunk (l & 15) ^ rr: the swizzle is applied on the global side.  Page ids come from a lane-wise
+  // global chunk (l & 15) ^ rr (V: ^ v_swz(rr)): the swizzle is applied on the global side.  Page ids come from a lane-wise
   // window (lane i = table entry pwin_base + i), read with v_readlane; it is refilled once per 64 pages.
   static_assert(kKT == 32, "the copy assignment below is for 2 groups per tile");
   constexpr int kGroupsPerWave = 4 / kQW;
@@ -356,11 +364,13 @@ void prefill_kernel(const PrefillArgs a) {
     }
     return make_rsrc(base + (ok ? off : 0) + (int64_t)g * c_sh, ok ? (uint32_t)(((nv - 1) * c_st + kD) * 2) : 0u);
   };
+  const int swz_shift = copies_k ? 0 : 1, swz_mask = copies_k ? 15 : 14;
   uint32_t dma_off[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int rr = 4 * i + (lane >> 4);
-    dma_off[i] = (uint32_t)((rr * c_st + 8 * ((lane & 15) ^ rr)) * 2);
+    // rr, or v_swz(rr) = 2 (rr & 7): a shift and a mask, both uniform
+    dma_off[i] = (uint32_t)((rr * c_st + 8 * ((lane & 15) ^ ((rr << swz_shift) & swz_mask))) * 2);
   }
   // i: the team's i-th tile.  Tile 0 (first = true) takes its first group's page id from the scalar load above.
   auto issue = [&](int i, uint8_t* Kst, uint8_t* Vst, bool first = false) __attribute__((always_inline)) {
@@ -392,7 +402,7 @@ void prefill_kernel(const PrefillArgs a) {
   for (int kk = 0; kk < 4; ++kk) k_rd[kk] = (uint32_t)(col * kRowB + (((4 * kk + g4) ^ col) << 4));
   const int rsw = 4 * g4 + ((lane & 15) >> 2);
   const int c_lo = ((lane & 15) & 3) >> 1;
-  const uint32_t v_rd = (uint32_t)(rsw * kRowB + (lane & 1) * 8);
+  uint32_t v_rd[8];  // filled below, beside tile 0's copies
 
   f32x4_t acc[kG][8];
 #pragma unroll
@@ -420,6 +430,17 @@ void prefill_kernel(const PrefillArgs a) {
           st[hh][kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv, qb[hh][kk], st[hh][kb], 0, 0, 0);
       }
     }
+    // Instruction order of the block above: four K operands ahead, then two MFMAs and one operand in turn.  Measured with
+    // the order of the P.V block below (us per call in a graph, before / V swizzle / these orders): 16 x U[512, 2048] 133.3 /
+    // 129.9 / 128.5, 64 x U[150, 400] 45.6 / 44.9 / 44.2, 1 x 300 10.7 / 10.9 / 10.3; two operands ahead 129.2 on the first, all
+    // eight 131.4.
+    __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 4, 0);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      __builtin_amdgcn_sched_group_barrier(kSchedMfma, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(kSchedMfma, 8, 0);
     // Mask: key j is visible to this lane's token iff j <= jlim (= min(Lk - 1, qpos) when causal).
     // Relative to the tile and this lane's key rows that is one compare per score against `lim`.
     // Masked scores become -inf; the running max m is kept in scaled (log2) units.
@@ -488,17 +509,26 @@ void prefill_kernel(const PrefillArgs a) {
     // operand's key order) comes from two transpose reads; each is used for both heads.
 #pragma unroll
     for (int db = 0; db < 8; ++db) {
-      const uint32_t chunk = (uint32_t)((((2 * db) + c_lo) ^ rsw) << 4);
 #pragma unroll
       for (int s2 = 0; s2 < kKT / 32; ++s2) {
-        const uint2 lo = ldtr(Vs + v_rd + chunk + (32 * s2) * kRowB);
-        const uint2 hi = ldtr(Vs + v_rd + chunk + (32 * s2 + 16) * kRowB);
+        const uint2 lo = ldtr(Vs + v_rd[db] + (32 * s2) * kRowB);
+        const uint2 hi = ldtr(Vs + v_rd[db] + (32 * s2 + 16) * kRowB);
         const bf16x8_t va = as_bf16x8(make_uint4(lo.x, lo.y, hi.x, hi.y));
 #pragma unroll
         for (int hh = 0; hh < kG; ++hh)
           acc[hh][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb[hh][s2], acc[hh][db], 0, 0, 0);
       }
     }
+    // Instruction order of the block above: two operands' reads ahead, then two MFMAs and one operand's reads in turn.
+    // (Left to itself the compiler reads two operands, waits for both, and leaves the LDS latency in the open;
+    // one operand ahead measured 133.8 us on 16 x U[512, 2048], three 134.4, two 130.0.)
+    __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 4, 0);
+#pragma unroll
+    for (int n = 0; n < 6; ++n) {
+      __builtin_amdgcn_sched_group_barrier(kSchedMfma, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(kSchedMfma, 4, 0);
   };
 
   // Stage (t+1) & 1 is filled while tile t is read from stage t & 1; the barrier at the end of each tile both
@@ -506,6 +536,9 @@ void prefill_kernel(const PrefillArgs a) {
   // The wait is unconditional so that no path into the loop carries outstanding loads (the q fragments): a
   // pending load on any entry path makes the compiler drain every copy before the first MFMA of each tile.
   if (ntiles > 0) issue(0, sK0, sV0, true);
+#pragma unroll
+  for (int db = 0; db < 8; ++db)
+    v_rd[db] = (uint32_t)(rsw * kRowB + (lane & 1) * 8 + (((2 * db + c_lo) ^ v_swz(rsw)) << 4));
   wait_vmem();
   __syncthreads();
   if constexpr (kRopeQ) {
@@ -609,7 +642,8 @@ void prefill_kernel(const PrefillArgs a) {
         const int row = key & (kKT - 1);
         const bool odd = (t / kS) & 1;  // tile t: stage (t / kS) & 1 of team t mod kS
         const uint8_t* stg = part == 0 ? (odd ? sK1 : sK0) : (odd ? sV1 : sV0);
-        const uint4 x = ld16(stg + (t % kS) * kTileB + row * kRowB + ((ch ^ (row & 15)) << 4));
+        const uint4 x = ld16(stg + (t % kS) * kTileB + row * kRowB +
+                             ((ch ^ (part == 0 ? row & 15 : v_swz(row))) << 4));
         uint16_t* dst = (part == 0 ? a.pk : a.pv) + (int64_t)page * a.p_sp +
                         (int64_t)(key & ((1 << a.p_shift) - 1)) * a.p_st + (int64_t)g * a.p_sh + 8 * ch;
         st16(dst, x);
