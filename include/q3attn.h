@@ -199,7 +199,7 @@ int q3a_paged_decode_append_rope(const void* q, int64_t q_stride_b, int64_t q_st
  * whose workspace (q3a_paged_decode_workspace_bytes) exceeds it are rejected with Q3A_ESPACE; every stream-K call
  * (split_tokens == 0, batch <= 4096) fits on MI355X.  All calls on one GPU share that array: calls that overlap on one
  * GPU (two streams at once) race, calls ordered on one stream do not.  Arguments, semantics and results are those of
- * q3a_paged_decode, bit for bit.
+ * q3a_paged_decode given that array as its workspace, bit for bit (5 to 64 rows: the balanced form where it applies).
  */
 int q3a_paged_decode_noalloc(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void* k_cache,
                              const void* v_cache, int64_t kv_stride_page, int64_t kv_stride_tok,
