@@ -1308,7 +1308,7 @@ static int resident_slots() {
 // the wider prologue, about 1 us.  Four teams of 32 query tokens where they fit, else two of 64.  us per call in a
 // graph, unsplit / split:
 //   packed (the keys are bounded by the longest query range; half of the query tiles see fewer)
-//     1 x 300 8.7 / 9.2, 1 x 400 12.3 / 10.6, 1 x 1,000 24.9 / 16.5, 1 x 2,048 (two teams) 46.2 / 36.4, 2 x 500 15.6 / 12.5
+//     1 x 200 8.4 / 9.2, 1 x 400 12.3 / 10.6, 1 x 1,000 24.9 / 16.5, 1 x 2,048 (two teams) 46.2 / 36.4, 2 x 500 15.6 / 12.5
 //   dense (every query tile sees the prefix): 8 x 100 + 50 8.3 / 9.9, 1 x 200 + 100 11.4 / 10.6, 4 x 250 + 150 14.9 / 12.9,
 //     6 x 210 + 170 (two teams) 14.8 / 13.6; two teams below that: 4 x U[150, 400] packed 13.3 / 12.9, 8 x U[150, 250] 18.4 / 19.6
 static int key_split(int num_seqs, int hkv, int max_seqlen_q, bool dense, int seqlen_k) {
