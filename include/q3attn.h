@@ -76,11 +76,11 @@ const char* q3a_last_error(void);
  * no tokens.  Requirements: D == 128, Hq == 2*Hkv, 1 <= Hkv <= 16, page_size % 16 == 0,
  * 16-byte aligned rows.  split_tokens == 0 lets the library choose the decomposition from the batch and
  * the table capacity max_pages_per_seq*page_size (never from the device-resident lengths): tables of at most
- * 256 tokens (above 64 rows: 128) and batches of 17 to 64 rows with tables of at most 2,048 tokens take
- * Q3A_DECODE_ROW, longer tables of at most 16 rows Q3A_DECODE_CHUNKS.  Of these, 5 to 16 rows of tables up to 2,048
- * tokens, 17 to 64 rows of tables from 528 tokens and 25 to 32 from 1,040 (above 16 rows at most 8 KV heads) are cut into
- * chunks on the device from the rows' lengths, so that they fill it once (the balanced form), where the workspace
- * holds q3a_paged_decode_workspace_bytes(..., Q3A_WORKSPACE_BALANCED) bytes.  Larger batches take stream-K (a persistent grid sized to the device, balanced over all rows' 16-token tiles; batch <= 4096,
+ * 128 tokens and batches of 17 to 64 rows with tables of at most 2,048 tokens take Q3A_DECODE_ROW, longer tables of at most
+ * 16 rows Q3A_DECODE_CHUNKS; of these, tables of 256 tokens take the one-launch kernel all the same (with the workspace of
+ * the chunks) and 5 to 16 rows of tables up to 2,048 tokens are cut into chunks on the device from the rows' lengths, so
+ * that they fill it once (the balanced form, in the same workspace).  Larger batches take stream-K (a persistent grid
+ * sized to the device, balanced over all rows' 16-token tiles; batch <= 4096,
  * larger batches fall back to q3a_paged_decode_default_split()).  The path codes above force one of them;
  * split_tokens > 0 (a multiple of 16, <= 1024) selects one workgroup per (row, split of that many tokens).
  */
@@ -198,8 +198,9 @@ int q3a_paged_decode_append_rope(const void* q, int64_t q_stride_b, int64_t q_st
  * The workspace is a static 8 MiB device array inside the library, one per GPU, held until the process ends.  Shapes
  * whose workspace (q3a_paged_decode_workspace_bytes) exceeds it are rejected with Q3A_ESPACE; every stream-K call
  * (split_tokens == 0, batch <= 4096) fits on MI355X.  All calls on one GPU share that array: calls that overlap on one
- * GPU (two streams at once) race, calls ordered on one stream do not.  Arguments, semantics and results are those of
- * q3a_paged_decode given that array as its workspace, bit for bit (5 to 64 rows: the balanced form where it applies).
+ * GPU (two streams at once) race, calls ordered on one stream do not.  Shapes that need no workspace (the query answers
+ * 0: 17 to 64 rows of up to 2,048 tokens among them) never touch it.  Arguments, semantics and results are those of
+ * q3a_paged_decode given that array as its workspace, bit for bit.
  */
 int q3a_paged_decode_noalloc(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void* k_cache,
                              const void* v_cache, int64_t kv_stride_page, int64_t kv_stride_tok,
@@ -209,9 +210,6 @@ int q3a_paged_decode_noalloc(const void* q, int64_t q_stride_b, int64_t q_stride
                              int head_dim, float softmax_scale, int split_tokens, void* stream);
 
 /* Bytes of workspace q3a_paged_decode needs for this shape and split (0 if none is needed). */
-/* As split_tokens of q3a_paged_decode_workspace_bytes() only: the bytes with which a call of split_tokens 0 may take the
- * balanced form (for shapes it does not serve, the bytes of split_tokens 0). */
-#define Q3A_WORKSPACE_BALANCED (-5)
 size_t q3a_paged_decode_workspace_bytes(int batch, int num_q_heads, int num_kv_heads, int head_dim,
                                         int max_pages_per_seq, int page_size, int split_tokens);
 

@@ -1530,7 +1530,7 @@ constexpr int row_max_waves(bool multi) { return multi ? kRowMaxWaves / 2 : kRow
 constexpr int kChunkMax = 16;  // records per (row, KV head): the combine loads them all at once
 
 //
-// Balanced form (kBal), for kBalMinBatch..kBalMaxBatch rows: the chunks are cut from the lengths the call finds on
+// Balanced form (kBal), for kBalMinBatch..kChunkMaxBatch rows: the chunks are cut from the lengths the call finds on
 // the device, not from the table capacity.  Each workgroup (4 waves) loads every row's length (one lane a row), derives
 // the same chunk length from their total, so that the rows' chunks together are about the workgroups the device
 // holds at once.  Workgroup b < batch takes row b's first chunk and loads its table entries and q beside the lengths;
@@ -1959,33 +1959,19 @@ bool chunk_geometry(int64_t cap_tiles, int* W, int* per, int* nch) {
 constexpr int kChunkMaxBatch = 16;
 constexpr int kChunkMinTiles = 2 * kMaxRowTiles;
 
-// The balanced form takes kBalMinBatch..kBalMaxBatch rows (a lane each) of tables up to 2,048 tokens, from 272 tokens
-// (up to 16 rows) or 528 (more rows, at most 8 KV heads).  Norm/rope form, us per call in a graph of 28, against the form
-// that served the shape before:
-//   below 5 rows the chunks are few and the extra round trip shows (chunks / balanced: 1 x 1,000 8.3 / 8.6,
-//     4 x 1,000 10.0 / 10.1); 5 to 16 rows: 16 x U[300, 1020] 18.7 / 14.9, 8 x U[900, 1780] 19.0 / 15.5, 8 x 500 9.9 / 9.9
+// The balanced form takes kBalMinBatch..kChunkMaxBatch rows (a lane each) of tables of 272 to 2,048 tokens, in place of the
+// chunked form and in its workspace.  Norm/rope form, us per call in a graph of 28 (chunks / balanced):
+//   below 5 rows the chunks are few and the extra round trip shows (1 x 1,000 8.3 / 8.6, 4 x 1,000 10.0 / 10.1);
+//     16 x U[300, 1020] 18.7 / 14.9, 8 x U[900, 1780] 19.0 / 15.5, 8 x 500 9.9 / 9.9
 //   two tiles a wave (tables of 256 tokens) are one launch of the row kernel: 8 x U[50, 250] 8.4 in chunks, 7.8
-//   17 to 64 rows (row kernel / balanced): 24 rows log-uniform in [178, 1780] 26.1 / 19.7, 64 46.4 / 38.4, 20 x U[500, 1000]
-//     18.9 / 17.4, 40 x U[890, 1780] 46.1 / 41.4.  Up to 512 tokens the row kernel's single launch wins (24 x 490 13.3 / 15.4),
-//     and up to 1,024 where its workgroups fill the CUs once (25 to 32 rows: 28 x U[500, 1000] 21.8 / 22.7, log-uniform in
-//     [100, 1000] 18.5 / 17.0).  Rows of nearly one length (within 5 %) lose the combine launch: 24 x 975 21.6 / 23.3,
-//     28 x 1,735 38.7 / 40.8, 64 x 1,735 74.5 / 78.6; the host does not know the lengths, and ragged rows are the rule.
+// 17 to 64 rows keep the row kernel's one launch, which needs no workspace: the second launch costs short rows in long
+// tables more than even chunks give long ones (row kernel / balanced, 2,048-token tables: 24 x U[20, 200] 8.4 / 10.7,
+// 32 x U[20, 200] 8.0 / 11.0, 28 x U[1946, 2048] 40.6 / 46.7).
 constexpr int kRowOneTiles = 16;
 constexpr int kBalMinBatch = 5;
-constexpr int kBalMaxBatch = 64;
-
-bool balanced_ok(int batch, int hkv, int64_t max_ctx) {
-  const int64_t cap_tiles = (max_ctx + kTile - 1) / kTile;
-  if (batch < kBalMinBatch || batch > kBalMaxBatch || cap_tiles > kRowMaxWaves * kRowMaxPer) return false;
-  if (batch <= kChunkMaxBatch) return cap_tiles > kRowOneTiles;
-  const int cu_rows = bal_resident(hkv) / 4;  // rows whose workgroups in the row kernel are one per CU
-  const bool fills = batch <= cu_rows && 4 * batch > 3 * cu_rows;
-  return hkv <= 8 && cap_tiles > (fills ? 4 : 2) * kRowOneTiles;
-}
-
-// Its shortest chunk (tiles): two tiles a wave, so a 2,048-token row has at most kChunkMax records and up to 16 rows
-// need no more workspace than their 128-token chunks; more rows than 32 fill the device with twice that.
-int bal_min_tiles(int batch) { return batch <= 32 ? 8 : 16; }
+// Its shortest chunk (tiles): two tiles a wave, so a 2,048-token row has at most kChunkMax records and the balanced form
+// needs no more workspace than 128-token chunks.
+constexpr int kBalMinTiles = 8;
 
 Path choose_path(int batch, int64_t max_ctx, int split_tokens) {
   const int64_t cap_tiles = (max_ctx + kTile - 1) / kTile;
@@ -2011,11 +1997,6 @@ Path choose_path(int batch, int64_t max_ctx, int split_tokens) {
 
 size_t workspace_bytes(int batch, int hkv, int max_pages, int page_size, int split_tokens) {
   const int64_t max_ctx = (int64_t)max_pages * page_size;
-  if (split_tokens == Q3A_WORKSPACE_BALANCED) {
-    if (balanced_ok(batch, hkv, max_ctx))
-      return (size_t)batch * ceil_div(ceil_div(max_ctx, kTile), bal_min_tiles(batch)) * hkv * kRowRec * sizeof(float);
-    split_tokens = 0;
-  }
   switch (choose_path(batch, max_ctx, split_tokens)) {
     case Path::kNone:
     case Path::kBalanced:  // never choose_path's
@@ -2239,18 +2220,13 @@ static int launch_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
   const int64_t max_ctx = (int64_t)max_pages_per_seq * page_size;
   if (max_ctx > (int64_t)1 << 30) return fail(Q3A_EINVAL, "%s: context capacity too large", who);
   Path path = choose_path(batch, max_ctx, split_tokens);
-  const bool bal_fits = balanced_ok(batch, num_kv_heads, max_ctx);
-  if (split_tokens == 0) {
-    // The balanced form where the workspace holds its records; a table of two tiles a wave takes the row kernel
-    // whatever the batch (the workspace stays that of the chunks).
-    if (bal_fits && workspace != nullptr && (uintptr_t)workspace % 16 == 0 &&
-        workspace_bytes_ >= workspace_bytes(batch, num_kv_heads, max_pages_per_seq, page_size, Q3A_WORKSPACE_BALANCED))
+  const int workspace_split = split_tokens;  // the value the caller sized the workspace with
+  if (split_tokens == 0 && path == Path::kChunks) {
+    if (max_ctx <= kRowOneTiles * kTile)
+      path = Path::kRow;  // two tiles a wave, one launch
+    else if (batch >= kBalMinBatch && max_ctx <= kRowMaxWaves * kRowMaxPer * kTile)
       path = Path::kBalanced;
-    else if (path == Path::kChunks && max_ctx <= kRowOneTiles * kTile)
-      path = Path::kRow;
   }
-  // The value the caller sized the workspace with.
-  const int workspace_split = path == Path::kBalanced ? Q3A_WORKSPACE_BALANCED : split_tokens;
   if (path == Path::kNone)
     return fail(Q3A_EINVAL, "%s: decode path %d does not take this shape (batch %d, table of %lld tokens)", who,
                 split_tokens, batch, (long long)max_ctx);
@@ -2266,7 +2242,7 @@ static int launch_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
   if (chunks) chunk_geometry(cap_tiles, &row_waves, &chunk_per, &nchunks);
   if (row) split_tokens = cap_tiles * kTile;
   if (chunks) split_tokens = row_waves * chunk_per * kTile;
-  if (bal) split_tokens = bal_min_tiles(batch) * kTile;
+  if (bal) split_tokens = kBalMinTiles * kTile;
   const bool sk = path == Path::kStreamK;
   if (sk) split_tokens = 0;
   if (path == Path::kFixed && split_tokens == 0)
@@ -2437,11 +2413,9 @@ static int launch_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
   a.ws = static_cast<float*>(workspace);
   if (bal) {
     // a.grid: chunks per KV head to aim for, short of the resident workgroups by half the batch (a row's chunks are
-    // rounded up).  More than 32 rows have one or two chunks each there, too coarse to even the CUs out: they aim for
-    // twice as many (64 x U[500, 1000] 41.7 -> 39.8 us per call, 64 x U[890, 1780] 67.3 -> 62.9; up to 32 rows 24.2 -> 26.1
-    // the other way).  The chunk length is at least total / a.grid, so the chunks number at most a.grid + batch.
-    a.row_per = bal_min_tiles(batch);
-    a.grid = std::max(1, (batch > 32 ? 2 : 1) * bal_resident(num_kv_heads) - batch / 2);
+    // rounded up).  The chunk length is at least total / a.grid, so the chunks number at most a.grid + batch.
+    a.row_per = kBalMinTiles;
+    a.grid = std::max(1, bal_resident(num_kv_heads) - batch / 2);
     const dim3 bgrid(num_kv_heads, std::min(a.grid + batch, batch * max_splits)), bblock(64 * kBalWaves);
     if (rope)
       hipLaunchKernelGGL((paged_decode_row_kernel<true, true, true, true>), bgrid, bblock, 0, st, a);

@@ -27,9 +27,6 @@ DECODE_ROW = -1        # one workgroup per (row, KV head), one launch (tables <=
 DECODE_CHUNKS = -2     # chunks of each row over many workgroups, then a combine (small batches of long rows)
 DECODE_STREAMK = -3    # stream-K over all rows' tiles, then a combine (batch <= 4096)
 DECODE_PLANNED = -4    # stream-K read from a per-frame plan (decode_plan); the plan is the call's workspace
-# Asks q3a_paged_decode_workspace_bytes for the bytes with which split_tokens 0 may take the balanced form (chunks cut on
-# the device from the rows' lengths; 5 to 64 rows).
-_WORKSPACE_BALANCED = -5
 
 # Plan forms (include/q3attn.h): which entry point a plan serves.
 _PLAN_FORMS = {"plain": 0, "append": 1, "append_rope": 2}
@@ -141,7 +138,7 @@ def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
         ws, ws_bytes, split = _plan_ws(plan, q, "paged_decode")
     else:
         split = int(split_tokens)            # 0: the library's default decomposition (stream-K)
-        ws_bytes = L.q3a_paged_decode_workspace_bytes(B, Hq, Hkv, D, max_pages, page, split or _WORKSPACE_BALANCED)
+        ws_bytes = L.q3a_paged_decode_workspace_bytes(B, Hq, Hkv, D, max_pages, page, split)
         ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=q.device)
     rc = L.q3a_paged_decode(
         q.data_ptr(), q.stride(0), q.stride(1),
@@ -198,7 +195,7 @@ def paged_decode_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cac
         ws, ws_bytes, split = _plan_ws(plan, q, "paged_decode_append")
     else:
         split = int(split_tokens)
-        ws_bytes = L.q3a_paged_decode_workspace_bytes(B, Hq, Hkv, D, max_pages, page, split or _WORKSPACE_BALANCED)
+        ws_bytes = L.q3a_paged_decode_workspace_bytes(B, Hq, Hkv, D, max_pages, page, split)
         ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=q.device)
     rc = L.q3a_paged_decode_append(
         q.data_ptr(), q.stride(0), q.stride(1),
@@ -268,7 +265,7 @@ def paged_decode_append_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
         ws, ws_bytes, split = _plan_ws(plan, q, "paged_decode_append_rope")
     else:
         split = int(split_tokens)
-        ws_bytes = L.q3a_paged_decode_workspace_bytes(B, Hq, Hkv, D, max_pages, page, split or _WORKSPACE_BALANCED)
+        ws_bytes = L.q3a_paged_decode_workspace_bytes(B, Hq, Hkv, D, max_pages, page, split)
         ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=dev)
     rc = L.q3a_paged_decode_append_rope(
         q.data_ptr(), q.stride(0), q.stride(1),

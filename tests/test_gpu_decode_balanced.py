@@ -1,13 +1,14 @@
-"""GPU parity of the balanced decode (the library's own choice for 5 to 64 rows): chunks cut on the
-device from all rows' lengths.
+"""GPU parity of the decode of small batches (the library's own choice for up to 64 rows; 5 to 16 rows: chunks cut on
+the device from all rows' lengths, 17 to 64: the row kernel).
 
 * against the oracle (bf16 output within max-abs 2e-2 and mean-abs 2e-3 of the fp32-softmax restatement of
-  engine/talker.py:82-88) at the edges of its range: the smallest and largest batch and table, one lane short of a wave,
+  engine/talker.py:82-88) at the edges of the ranges: the smallest and largest batch and table, one lane short of a wave,
   rows of 0, 1, a tile, a tile and a token, and full tables, all rows full (the longest chunks) and all rows empty but one;
 * the plain form bit-identical to the append form on the same tokens, and that with the norm/rope form on +-1 rows,
   whose normalised rows are exact (the same decomposition in all three);
-* the shapes just outside its range, against the oracle; a call whose workspace does not hold its records is the row
-  kernel's.
+* the shapes beside the ranges bit-identical to the path that serves them;
+* 17 to 64 rows need no workspace (q3a_paged_decode_workspace_bytes of split_tokens 0 is 0) and so write none, whatever
+  buffer the call is handed: a caller may share it between streams.
 """
 import numpy as np
 import pytest
@@ -86,40 +87,56 @@ def test_balanced_rope_form_exact_rows(cuda_device):
     assert torch.equal(out, ref) and torch.equal(kc, wl.k_cache) and torch.equal(vc, wl.v_cache)
 
 
+ROW, CHUNKS, SK = q3attn.DECODE_ROW, q3attn.DECODE_CHUNKS, q3attn.DECODE_STREAMK
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,cap", [(4, 1024), (65, 1024), (8, 256), (17, 512), (28, 1024), (8, 2064)])
-def test_shapes_beside_its_range(cuda_device, B, cap):
+@pytest.mark.parametrize("B,cap,path", [(4, 1024, CHUNKS), (65, 1024, SK), (8, 256, ROW), (17, 512, ROW), (17, 528, ROW),
+                                        (28, 1024, ROW), (33, 2048, ROW), (64, 2048, ROW), (8, 2064, CHUNKS)])
+def test_shapes_beside_its_range(cuda_device, B, cap, path):
     wl = W.make_decode("bal_no", cuda_device, ctx=_ctx(max(B, 5), cap, "ragged")[:B], num_pages=4 * B * 130, max_ctx=cap, seed=B)
     L = wl.layers[0]
     out = q3attn.paged_decode(L.q, wl.k_cache, wl.v_cache, wl.cache_seqlens, L.block_table, wl.scale)
     ok, st = ora.compare(to_np(out), decode_oracle(wl))
     assert ok, st
+    forced = q3attn.paged_decode(L.q, wl.k_cache, wl.v_cache, wl.cache_seqlens, L.block_table, wl.scale, path)
+    assert torch.equal(out, forced)
+
+
+def _c_decode(fn, wl, out, *ws):
+    L = wl.layers[0]
+    return fn(L.q.data_ptr(), L.q.stride(0), L.q.stride(1), wl.k_cache.data_ptr(), wl.v_cache.data_ptr(),
+              *wl.k_cache.stride()[:3], wl.k_cache.shape[0], wl.page_size, wl.cache_seqlens.data_ptr(),
+              L.block_table.data_ptr(), L.block_table.stride(0), L.block_table.shape[1], out.data_ptr(), out.stride(0),
+              out.stride(1), *ws, wl.batch, W.HQ, W.HKV, W.HEAD_DIM, wl.scale, 0, torch.cuda.current_stream().cuda_stream)
 
 
 @pytest.mark.gpu
-def test_without_the_workspace_the_row_kernel(cuda_device):
-    """17 to 64 rows need no workspace (q3a_paged_decode_workspace_bytes of split_tokens 0 is 0): without one the call is
-    the row kernel's, bit for bit."""
-    wl = W.make_decode("bal_ws", cuda_device, ctx=_ctx(20, 1024, "ragged"), num_pages=4096, max_ctx=1024, seed=3)
+@pytest.mark.parametrize("B,cap", [(17, 2048), (20, 1024), (33, 544), (64, 2048)])
+def test_no_workspace_is_touched_from_17_rows(cuda_device, B, cap):
+    """Without a workspace, with a large one (left as it was) and through the entry point that shares one array between
+    all its calls: the row kernel, bit for bit."""
+    wl = W.make_decode("bal_ws", cuda_device, ctx=_ctx(B, cap, "ragged"), num_pages=2 * B * (cap // 16 + 1), max_ctx=cap, seed=3)
     L, lib = wl.layers[0], _lib.lib()
-    out = torch.empty_like(L.q)
-    rc = lib.q3a_paged_decode(L.q.data_ptr(), L.q.stride(0), L.q.stride(1), wl.k_cache.data_ptr(), wl.v_cache.data_ptr(),
-                              *wl.k_cache.stride()[:3], wl.k_cache.shape[0], wl.page_size, wl.cache_seqlens.data_ptr(),
-                              L.block_table.data_ptr(), L.block_table.stride(0), L.block_table.shape[1], out.data_ptr(),
-                              out.stride(0), out.stride(1), None, 0, 20, W.HQ, W.HKV, W.HEAD_DIM, wl.scale, 0,
-                              torch.cuda.current_stream().cuda_stream)
-    assert rc == 0
-    row = q3attn.paged_decode(L.q, wl.k_cache, wl.v_cache, wl.cache_seqlens, L.block_table, wl.scale, q3attn.DECODE_ROW)
-    assert torch.equal(out, row)
+    row = q3attn.paged_decode(L.q, wl.k_cache, wl.v_cache, wl.cache_seqlens, L.block_table, wl.scale, ROW)
+    out = torch.full_like(L.q, float("nan"))
+    assert _c_decode(lib.q3a_paged_decode, wl, out, None, 0) == 0 and torch.equal(out, row)
+    arena = torch.full((8 << 20,), 0x5A, dtype=torch.uint8, device=cuda_device)
+    out.fill_(float("nan"))
+    assert _c_decode(lib.q3a_paged_decode, wl, out, arena.data_ptr(), arena.numel()) == 0 and torch.equal(out, row)
+    assert bool((arena == 0x5A).all())
+    out.fill_(float("nan"))
+    assert _c_decode(lib.q3a_paged_decode_noalloc, wl, out) == 0 and torch.equal(out, row)
 
 
 def test_workspace_query():
-    """The balanced form's records, 8 tiles a chunk (16 above 32 rows); elsewhere the bytes of split_tokens 0."""
+    """5 to 16 rows: the records of 128-token chunks; 17 to 64 rows of up to 2,048 tokens: none, for every head count."""
     ws = lambda B, pages, split, hkv=8: _lib.lib().q3a_paged_decode_workspace_bytes(B, 2 * hkv, hkv, 128, pages, 16, split)
-    assert ws(16, 128, -5) == ws(16, 128, 0) == 16 * 16 * 8 * 1040
-    assert ws(20, 65, -5) == 20 * 9 * 8 * 1040 and ws(64, 128, -5) == 64 * 8 * 8 * 1040
-    for B, pages, hkv in ((4, 128, 8), (65, 128, 8), (8, 16, 8), (17, 32, 8), (28, 64, 8), (8, 129, 8), (20, 65, 16)):
-        assert ws(B, pages, -5, hkv) == ws(B, pages, 0, hkv)
+    assert ws(16, 128, 0) == 16 * 16 * 8 * 1040 and ws(5, 17, 0) == 5 * 3 * 8 * 1040
+    for B in (17, 32, 33, 64):
+        for pages in (9, 16, 17, 33, 65, 128):
+            for hkv in (1, 8, 16):
+                assert ws(B, pages, 0, hkv) == 0
 
 
 def test_chunk_count_arithmetic():
