@@ -263,6 +263,10 @@ __device__ __forceinline__ uint32_t u4get(const uint4& v, int c) {
 // bf16 pairs (tokens 0,1 and 2,3) and each output dim takes two dot2 against the matching V pairs
 // built with v_perm_b32, the rounding point flash-attention also uses for P.  The running max
 // rarely grows after the first tiles, so the rescale of (l, acc) runs only when a lane's max grew.
+// kP32: the probabilities stay in fp32 (4 x 8 dims x 2 heads of FMA against V's upper and lower halves), for the waves
+// that hold two tiles in one state where they had one each: rounded to bf16, p is exact only where it sets its
+// state's maximum, so fewer states over more tokens lost precision.
+template <bool kP32 = false>
 __device__ __forceinline__ void tile_update(const DecodeArgs& a, const TileList& L, const uint4 (&q)[kG],
                                             const KVTile& T, int j, int grp, float (&m)[kG],
                                             float (&l)[kG], float (&acc)[kG][8]) {
@@ -304,6 +308,29 @@ __device__ __forceinline__ void tile_update(const DecodeArgs& a, const TileList&
 #pragma unroll
       for (int d = 0; d < 8; ++d) acc[h][d] *= alpha;
     }
+  }
+  if constexpr (kP32) {
+    float p[kG][4];
+#pragma unroll
+    for (int h = 0; h < kG; ++h) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[h][i] = fast_exp2(sc[h][i] - m[h]);
+      l[h] += (p[h][0] + p[h][1]) + (p[h][2] + p[h][3]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint32_t vw = u4get(T.v[i], c);
+        const float v0 = __uint_as_float(vw << 16), v1 = __uint_as_float(vw & 0xFFFF0000u);
+#pragma unroll
+        for (int h = 0; h < kG; ++h) {
+          acc[h][2 * c] = fmaf(p[h][i], v0, acc[h][2 * c]);
+          acc[h][2 * c + 1] = fmaf(p[h][i], v1, acc[h][2 * c + 1]);
+        }
+      }
+    }
+    return;
   }
   // V pairs: vp[pair][c][0] = (v[2*pair][dim 2c], v[2*pair+1][dim 2c]), [1] for dim 2c+1.
   uint32_t vp[2][4][2];
@@ -1530,42 +1557,18 @@ constexpr int row_max_waves(bool multi) { return multi ? kRowMaxWaves / 2 : kRow
 constexpr int kChunkMax = 16;  // records per (row, KV head): the combine loads them all at once
 
 //
-// Balanced form (kBal), for kBalMinBatch..kChunkMaxBatch rows: the chunks are cut from the lengths the call finds on
-// the device, not from the table capacity.  Each workgroup (4 waves) loads every row's length (one lane a row), derives
-// the same chunk length from their total, so that the rows' chunks together are about the workgroups the device
-// holds at once.  Workgroup b < batch takes row b's first chunk and loads its table entries and q beside the lengths;
-// the others find their (row, chunk >= 1) by a scan and a ballot, one more round trip, or exit past the last one.
-constexpr int kBalWaves = 4;
+// Listed form (kListed) of 128-token chunks, for grids that would otherwise be more than one workgroup a CU: 4 waves of two
+// tiles (kP32), and only chunks that hold tokens are spread over the CUs.  Workgroup b < batch takes row b's first
+// chunk, its loads in one trip; the others find their (row, chunk >= 1) from all rows' lengths (a lane each) by a scan
+// and a ballot, one more trip, or exit past the last one.  The chunks are cut from each row alone, so a row's result does not
+// depend on its neighbours.
+constexpr int kListedWaves = 4;
 
-struct BalSplit {
-  int ctx, n, nch;  // lane i: row i's context, tiles and chunks (at least 1 for a row of the batch: it writes zeros)
-};
-
-// The rows' cache_seqlens, lane i row i's (past the batch: the last row's, which balanced_split drops).
-__device__ __forceinline__ int balanced_seqlens(const DecodeArgs& a, int lane) { return a.seqlens[min(lane, a.batch - 1)]; }
-
-// ceil(n / d) for 0 <= n < 2^20, 1 <= d: the quotient is at least 1 / (2 d) away from the next integer, far more than
-// the reciprocal's error.
-__device__ __forceinline__ int ceil_div_small(int n, int d) {
-  return (int)(((float)(n + d) - 0.5f) * __builtin_amdgcn_rcpf((float)d));
-}
-
-template <bool kAppend>
-__device__ __forceinline__ BalSplit balanced_split(const DecodeArgs& a, int c, int lane) {
-  BalSplit s;
-  s.ctx = lane < a.batch ? ctx_of<kAppend>(c, a.max_pages * a.page_size) : 0;
-  s.n = (s.ctx + kTile - 1) / kTile;
-  const int total = readlane(wave_scan_incl(s.n), 63);
-  const int ct = max(a.row_per, __builtin_amdgcn_readfirstlane(ceil_div_small(total, a.grid)));
-  s.nch = lane < a.batch ? max(1, ceil_div_small(s.n, ct)) : 0;
-  return s;
-}
-
-template <bool kAppend, bool kMulti, bool kRope = false, bool kBal = false>
-__global__ __launch_bounds__(64 * (kBal ? kBalWaves : row_max_waves(kMulti)), kBal ? 4 : 1)
+template <bool kAppend, bool kMulti, bool kRope = false, bool kListed = false>
+__global__ __launch_bounds__(64 * (kListed ? kListedWaves : row_max_waves(kMulti)), kListed ? 4 : 1)
 void paged_decode_row_kernel(const DecodeArgs a) {
   static_assert(kAppend || !kRope, "the norm/rope form is an append form");
-  constexpr int kWaves = kBal ? kBalWaves : kRowMaxWaves;
+  constexpr int kWaves = kListed ? kListedWaves : kRowMaxWaves;
   __shared__ __align__(16) float rec[kWaves][kRowRec];
   __shared__ __align__(16) uint4 snew[kAppend ? kWaves : 1][2][kD / 8];  // per wave: the new k and v rows
   // The KV head is the fastest grid dimension: workgroups go to the XCDs in launch order, so with 8 heads every XCD
@@ -1573,32 +1576,24 @@ void paged_decode_row_kernel(const DecodeArgs a) {
   // longest rows decided the call.
   const int g = blockIdx.x;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int W = kBal ? kBalWaves : (int)(blockDim.x >> 6);
+  const int W = kListed ? kListedWaves : (int)(blockDim.x >> 6);
   const int lane = threadIdx.x & 63;
   const int grp = lane >> 4;
   const int dl = (lane & 15) * 8;
-  int b = blockIdx.y, ch = 0, CT = 0, ctx = 0, nch = 0;  // row, chunk, tiles per chunk, the row's context and chunks
-  int c_row = 0;
-  // Row r's context, chunks and (equal) chunk length from the split of all rows.
-  auto take = [&](const BalSplit& s, int r) __attribute__((always_inline)) {
-    ctx = readlane(s.ctx, r);
-    nch = readlane(s.nch, r);
-    CT = max(1, __builtin_amdgcn_readfirstlane(ceil_div_small(readlane(s.n, r), nch)));
-  };
-  if constexpr (kBal) {
-    c_row = balanced_seqlens(a, lane);
+  const int CT = W * a.row_per;  // tiles per chunk (the one-launch path: the whole table)
+  const int cap = a.max_pages * a.page_size;
+  int b = blockIdx.y, ch = blockIdx.z;
+  if constexpr (kListed) {
     if (b >= a.batch) {
       const int extra = b - a.batch;  // this workgroup's place among the rows' chunks 1, 2, ...
-      const BalSplit s = balanced_split<kAppend>(a, c_row, lane);
-      const int incl = wave_scan_incl(max(s.nch - 1, 0));
+      const int c = a.seqlens[min(lane, a.batch - 1)];
+      const int n = lane < a.batch ? (ctx_of<kAppend>(c, cap) + kTile - 1) / kTile : 0;
+      const int more = n > CT ? (n + CT - 1) / CT - 1 : 0;  // row `lane`'s chunks past its first
+      const int incl = wave_scan_incl(more);
       if (extra >= readlane(incl, 63)) return;  // uniform over the workgroup
       b = __builtin_popcountll(__ballot(incl <= extra));
-      take(s, b);
-      ch = extra - (readlane(incl, b) - nch);
+      ch = 1 + extra - (readlane(incl, b) - readlane(more, b));
     }
-  } else {
-    ch = blockIdx.z;
-    CT = W * a.row_per;  // the one-launch path: the whole table
   }
   const int tb = ch * CT;  // first tile of this workgroup's chunk
 
@@ -1610,8 +1605,7 @@ void paged_decode_row_kernel(const DecodeArgs a) {
   __asm__ volatile("" ::"s"(a.seqlens), "s"(a.bt), "s"(a.bt_sb), "s"(a.max_pages), "s"(a.page_size), "s"(a.row_per),
                    "s"(a.q), "s"(a.q_sb), "s"(a.q_sh), "s"(a.scale_log2), "s"(a.kc), "s"(a.vc), "s"(a.kv_sp),
                    "s"(a.kv_st), "s"(a.kv_sh));
-  if constexpr (!kBal) c_row = a.seqlens[b];
-  const int cap = a.max_pages * a.page_size;
+  const int c_row = a.seqlens[b];
   const int t = kTile * (tb + w + lane * W);  // first token of this lane's tile
   const int pidx = min(t, cap - 1) / a.page_size;
   const int page = a.bt[(int64_t)b * a.bt_sb + pidx];
@@ -1641,16 +1635,12 @@ void paged_decode_row_kernel(const DecodeArgs a) {
       snew[w][1][lane] = vn;
     }
   }
-  if constexpr (kBal) {
-    if (ch == 0) take(balanced_split<kAppend>(a, c_row, lane), b);
-  } else {
-    ctx = ctx_of<kAppend>(c_row, cap);
-  }
+  const int ctx = ctx_of<kAppend>(c_row, cap);
   const int nrow = (ctx + kTile - 1) / kTile;  // tiles of the row
-  if constexpr (!kBal) nch = (nrow + CT - 1) / CT;  // chunks holding tiles of the row
+  const int nch = (nrow + CT - 1) / CT;        // chunks holding tiles of the row
   // Chunks past the row's end have nothing to do (chunk 0 stays: it writes the zero row of an empty one).  The
   // condition is uniform over the workgroup.
-  if (!kBal && ch > 0 && ch >= nch) return;
+  if (ch > 0 && ch >= nch) return;
   const int nrc = min(nrow - tb, CT);          // tiles of the row in this chunk
 
   TileList L;
@@ -1686,7 +1676,7 @@ void paged_decode_row_kernel(const DecodeArgs a) {
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    tile_update(a, L, q, T, j, grp, m, l, acc);
+    tile_update<kListed>(a, L, q, T, j, grp, m, l, acc);
   };
 
   if constexpr (!kMulti) {
@@ -1740,7 +1730,7 @@ void paged_decode_row_kernel(const DecodeArgs a) {
   const int d0 = (lane & 31) * 4;
   // Each group's LDS reads are all in flight before the first is used, those of absent waves (inside the array, never
   // used) among them; a loop over the W states waited for two LDS latencies each.
-  constexpr int kU = kBal ? kBalWaves : 8;
+  constexpr int kU = kListed ? kListedWaves : 8;
   float M = kMaxSeed;
 #pragma unroll
   for (int v0 = 0; v0 < kWaves; v0 += kU) {
@@ -1798,11 +1788,7 @@ void paged_decode_row_kernel(const DecodeArgs a) {
 // 4*(l%32)..+4.  The records of every chunk of the grid are loaded at once, before the row's context is known (the
 // combine is one memory round trip); those of chunks past the row's end are stale and are never used.  Rows held by
 // one chunk were written by the row kernel.
-// The balanced form knows a row's chunks only from all lengths (one round trip): it loads kBalEager records beside
-// them and the rest of a row that has more after.
-constexpr int kBalEager = 4;
-
-template <bool kAppend, bool kBal = false>
+template <bool kAppend>
 __global__ __launch_bounds__(64) void paged_decode_chunk_combine_kernel(const DecodeArgs a) {
   const int b = blockIdx.y;
   const int g = blockIdx.x;
@@ -1813,30 +1799,21 @@ __global__ __launch_bounds__(64) void paged_decode_chunk_combine_kernel(const De
   const float* base = a.ws + ((int64_t)b * nchg * a.hkv + g) * kRowRec;
   uint4 o[kChunkMax];
   float mr[kChunkMax], lr[kChunkMax];
-  auto load = [&](int u, int n) __attribute__((always_inline)) {
+#pragma unroll
+  for (int u = 0; u < kChunkMax; ++u) {
     o[u] = make_uint4(0u, 0u, 0u, 0u);
     mr[u] = kMaxSeed;
     lr[u] = 0.f;
-    if (u < n) {
+    if (u < nchg) {
       const float* r = base + (int64_t)u * a.hkv * kRowRec;
       o[u] = ld16(r + h * kD + d0);
       mr[u] = r[kG * kD + h];
       lr[u] = r[kG * kD + kG + h];
     }
-  };
-  constexpr int kEager = kBal ? kBalEager : kChunkMax;
-  const int c_all = kBal ? balanced_seqlens(a, lane) : 0;
-#pragma unroll
-  for (int u = 0; u < kEager; ++u) load(u, nchg);
-  int nch;
-  if constexpr (kBal) {
-    nch = readlane(balanced_split<kAppend>(a, c_all, lane).nch, b);
-  } else {
-    nch = (row_ctx<kAppend>(a, b) + a.split_tokens - 1) / a.split_tokens;
   }
+  const int ctx = row_ctx<kAppend>(a, b);
+  const int nch = (ctx + a.split_tokens - 1) / a.split_tokens;
   if (nch <= 1) return;
-#pragma unroll
-  for (int u = kEager; u < kChunkMax; ++u) load(u, nch);
   float M = kMaxSeed;
 #pragma unroll
   for (int u = 0; u < kChunkMax; ++u)
@@ -1908,17 +1885,17 @@ int sk_grid_of(int hkv, int form) {
   return g;
 }
 
-// Workgroups per KV head of the balanced form the current device holds at once (4 waves a SIMD; cached per device).
-int bal_resident(int hkv) {
+// Compute units of the current device (cached per device).
+int num_cus() {
   static std::atomic<int> cache[64];
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256 * 4 / hkv;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
   int cus = cache[dev].load(std::memory_order_relaxed);
   if (cus <= 0) {
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 256 * 4 / hkv;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 256;
     cache[dev].store(cus, std::memory_order_relaxed);
   }
-  return cus * 4 / hkv;
+  return cus;
 }
 
 int sk_grid(int hkv) {
@@ -1934,7 +1911,7 @@ int sk_effective_grid_host(int grid, int64_t nt) {
 
 // The decompositions of one decode call.  split_tokens == 0 lets choose_path pick; Q3A_DECODE_ROW,
 // Q3A_DECODE_CHUNKS and Q3A_DECODE_STREAMK (negative codes) ask for one; split_tokens > 0 is the fixed split.
-enum class Path { kNone, kRow, kChunks, kBalanced, kStreamK, kFixed };
+enum class Path { kNone, kRow, kChunks, kStreamK, kFixed };
 
 // Chunked form geometry for a table of cap_tiles tiles: W waves of `per` tiles per chunk, nch chunks per row.
 // 128-token chunks (8 waves of one tile) while 16 of them cover the table, then 16 waves of one tile, then 8
@@ -1959,19 +1936,18 @@ bool chunk_geometry(int64_t cap_tiles, int* W, int* per, int* nch) {
 constexpr int kChunkMaxBatch = 16;
 constexpr int kChunkMinTiles = 2 * kMaxRowTiles;
 
-// The balanced form takes kBalMinBatch..kChunkMaxBatch rows (a lane each) of tables of 272 to 2,048 tokens, in place of the
-// chunked form and in its workspace.  Norm/rope form, us per call in a graph of 28 (chunks / balanced):
-//   below 5 rows the chunks are few and the extra round trip shows (1 x 1,000 8.3 / 8.6, 4 x 1,000 10.0 / 10.1);
-//     16 x U[300, 1020] 18.7 / 14.9, 8 x U[900, 1780] 19.0 / 15.5, 8 x 500 9.9 / 9.9
-//   two tiles a wave (tables of 256 tokens) are one launch of the row kernel: 8 x U[50, 250] 8.4 in chunks, 7.8
-// 17 to 64 rows keep the row kernel's one launch, which needs no workspace: the second launch costs short rows in long
-// tables more than even chunks give long ones (row kernel / balanced, 2,048-token tables: 24 x U[20, 200] 8.4 / 10.7,
-// 32 x U[20, 200] 8.0 / 11.0, 28 x U[1946, 2048] 40.6 / 46.7).
+// Small batches of 256-token tables: two tiles a wave are one launch of the row kernel.
 constexpr int kRowOneTiles = 16;
-constexpr int kBalMinBatch = 5;
-// Its shortest chunk (tiles): two tiles a wave, so a 2,048-token row has at most kChunkMax records and the balanced form
-// needs no more workspace than 128-token chunks.
-constexpr int kBalMinTiles = 8;
+
+// The listed form takes the place of 8-wave workgroups of 128-token chunks (tables up to 2,048 tokens) where their grid
+// of the table's capacity is more than one workgroup a CU and each row has a lane: below, the workgroups of absent chunks are
+// on CUs of their own, and the extra trip shows.  Us per call in a graph of 28, chunks of the capacity / listed:
+//   norm/rope: 8 x 512 (256 workgroups) 9.1 / 9.1 log-uniform, 9.0 / 9.3 U[205, 358]; 6 x U[384, 768] (288) 11.4 / 9.6;
+//     16 rows log-uniform in [64, 1280] 20.2 / 12.8, U[1946, 2048] 33.1 / 30.0; all shapes from 288 workgroups 0.40 to 1.01
+//   plain: 16 log-uniform in [64, 1280] 15.3 / 12.1, 6 x U[1024, 2048] 13.4 / 13.9 (the worst), the rest 0.54 to 1.03
+bool listed_chunks(int batch, int hkv, int row_waves, int row_per, int nchunks) {
+  return row_waves == 8 && row_per == 1 && batch <= 64 && (int64_t)batch * nchunks * hkv > num_cus();
+}
 
 Path choose_path(int batch, int64_t max_ctx, int split_tokens) {
   const int64_t cap_tiles = (max_ctx + kTile - 1) / kTile;
@@ -1999,7 +1975,6 @@ size_t workspace_bytes(int batch, int hkv, int max_pages, int page_size, int spl
   const int64_t max_ctx = (int64_t)max_pages * page_size;
   switch (choose_path(batch, max_ctx, split_tokens)) {
     case Path::kNone:
-    case Path::kBalanced:  // never choose_path's
     case Path::kRow: return 0;
     case Path::kChunks: {
       int w, p, n;
@@ -2221,28 +2196,21 @@ static int launch_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
   if (max_ctx > (int64_t)1 << 30) return fail(Q3A_EINVAL, "%s: context capacity too large", who);
   Path path = choose_path(batch, max_ctx, split_tokens);
   const int workspace_split = split_tokens;  // the value the caller sized the workspace with
-  if (split_tokens == 0 && path == Path::kChunks) {
-    if (max_ctx <= kRowOneTiles * kTile)
-      path = Path::kRow;  // two tiles a wave, one launch
-    else if (batch >= kBalMinBatch && max_ctx <= kRowMaxWaves * kRowMaxPer * kTile)
-      path = Path::kBalanced;
-  }
+  if (split_tokens == 0 && path == Path::kChunks && max_ctx <= kRowOneTiles * kTile) path = Path::kRow;
   if (path == Path::kNone)
     return fail(Q3A_EINVAL, "%s: decode path %d does not take this shape (batch %d, table of %lld tokens)", who,
                 split_tokens, batch, (long long)max_ctx);
-  // Narrow tables and small batches: one workgroup per (row, KV head) streams the row with up to 16 waves and
+  // Narrow tables and small batches: one workgroup per (row, KV head) streams the row with up to 8 waves and
   // writes its output, one kernel and no partial records.  Stream-K would cut such rows into short pieces and merge
   // them in a second kernel, whose launch is most of such a call.  Small batches of long rows: the same kernel over
   // chunks of the row, so the row's tiles spread over many CUs, and a combine.
   const bool row = path == Path::kRow;
   const bool chunks = path == Path::kChunks;
-  const bool bal = path == Path::kBalanced;
   const int cap_tiles = (int)((max_ctx + kTile - 1) / kTile);
   int row_waves = std::min(cap_tiles, kRowMaxWaves / 2), chunk_per = 1, nchunks = 1;
   if (chunks) chunk_geometry(cap_tiles, &row_waves, &chunk_per, &nchunks);
   if (row) split_tokens = cap_tiles * kTile;
   if (chunks) split_tokens = row_waves * chunk_per * kTile;
-  if (bal) split_tokens = kBalMinTiles * kTile;
   const bool sk = path == Path::kStreamK;
   if (sk) split_tokens = 0;
   if (path == Path::kFixed && split_tokens == 0)
@@ -2277,7 +2245,7 @@ static int launch_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
   }
   if (nr != nullptr) {
     if (!append) return fail(Q3A_EINVAL, "%s: the norm/rope form needs k_new/v_new", who);
-    if (!row && !sk && !chunks && !bal)
+    if (!row && !sk && !chunks)
       return fail(Q3A_EINVAL, "%s: the norm/rope form needs split_tokens <= 0 and batch <= %d", who, kSkMaxRows);
     if (sk && num_kv_heads > 8)
       return fail(Q3A_EINVAL, "%s: the norm/rope form supports at most 8 KV heads (got %d)", who, num_kv_heads);
@@ -2411,31 +2379,13 @@ static int launch_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
   a.grid = 0;
   a.prefix = nullptr;
   a.ws = static_cast<float*>(workspace);
-  if (bal) {
-    // a.grid: chunks per KV head to aim for, short of the resident workgroups by half the batch (a row's chunks are
-    // rounded up).  The chunk length is at least total / a.grid, so the chunks number at most a.grid + batch.
-    a.row_per = kBalMinTiles;
-    a.grid = std::max(1, bal_resident(num_kv_heads) - batch / 2);
-    const dim3 bgrid(num_kv_heads, std::min(a.grid + batch, batch * max_splits)), bblock(64 * kBalWaves);
-    if (rope)
-      hipLaunchKernelGGL((paged_decode_row_kernel<true, true, true, true>), bgrid, bblock, 0, st, a);
-    else if (append)
-      hipLaunchKernelGGL((paged_decode_row_kernel<true, true, false, true>), bgrid, bblock, 0, st, a);
-    else
-      hipLaunchKernelGGL((paged_decode_row_kernel<false, true, false, true>), bgrid, bblock, 0, st, a);
-    e = hipGetLastError();
-    if (e != hipSuccess) return fail(Q3A_ELAUNCH, "%s: balanced launch failed: %s", who, hipGetErrorString(e));
-    const dim3 cgrid(num_kv_heads, batch);
-    if (append)
-      hipLaunchKernelGGL((paged_decode_chunk_combine_kernel<true, true>), cgrid, dim3(64), 0, st, a);
-    else
-      hipLaunchKernelGGL((paged_decode_chunk_combine_kernel<false, true>), cgrid, dim3(64), 0, st, a);
-    e = hipGetLastError();
-    if (e != hipSuccess) return fail(Q3A_ELAUNCH, "%s: combine launch failed: %s", who, hipGetErrorString(e));
-    return Q3A_OK;
-  }
   if (row || chunks) {
     a.row_per = chunks ? chunk_per : (cap_tiles + row_waves - 1) / row_waves;
+    const bool listed = chunks && listed_chunks(batch, num_kv_heads, row_waves, chunk_per, nchunks);
+    if (listed) {
+      row_waves = kListedWaves;
+      a.row_per = 2;
+    }
     // The row is grid dimension y, which holds 65,535: larger batches go in slices of rows.
     constexpr int kGridRows = 65535;
     for (int row0 = 0; row0 < batch; row0 += kGridRows) {
@@ -2455,8 +2405,15 @@ static int launch_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
         }
         if (chunks && nchunks > 1) a.ws += (int64_t)kGridRows * nchunks * num_kv_heads * kRowRec;
       }
-      const dim3 rgrid(num_kv_heads, rows, chunks ? nchunks : 1), rblock(64 * row_waves);
-      if (a.row_per == 1) {
+      const dim3 rgrid(num_kv_heads, listed ? rows * nchunks : rows, chunks && !listed ? nchunks : 1), rblock(64 * row_waves);
+      if (listed) {
+        if (rope)
+          hipLaunchKernelGGL((paged_decode_row_kernel<true, true, true, true>), rgrid, rblock, 0, st, a);
+        else if (append)
+          hipLaunchKernelGGL((paged_decode_row_kernel<true, true, false, true>), rgrid, rblock, 0, st, a);
+        else
+          hipLaunchKernelGGL((paged_decode_row_kernel<false, true, false, true>), rgrid, rblock, 0, st, a);
+      } else if (a.row_per == 1) {
         if (rope)
           hipLaunchKernelGGL((paged_decode_row_kernel<true, false, true>), rgrid, rblock, 0, st, a);
         else if (append)

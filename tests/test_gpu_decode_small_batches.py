@@ -1,11 +1,12 @@
-"""GPU parity of the decode of small batches (the library's own choice for up to 64 rows; 5 to 16 rows: chunks cut on
-the device from all rows' lengths, 17 to 64: the row kernel).
+"""GPU parity of the decode of small batches (the library's own choice for up to 64 rows; up to 16 rows: 128-token
+chunks, listed from the rows' lengths where their grid is more than one workgroup a CU; 17 to 64: the row kernel).
 
 * against the oracle (bf16 output within max-abs 2e-2 and mean-abs 2e-3 of the fp32-softmax restatement of
   engine/talker.py:82-88) at the edges of the ranges: the smallest and largest batch and table, one lane short of a wave,
-  rows of 0, 1, a tile, a tile and a token, and full tables, all rows full (the longest chunks) and all rows empty but one;
+  rows of 0, 1, a tile, a tile and a token, and full tables, all rows full (the longest lists) and all rows empty but one;
 * the plain form bit-identical to the append form on the same tokens, and that with the norm/rope form on +-1 rows,
   whose normalised rows are exact (the same decomposition in all three);
+* a row's bits do not depend on the other rows' lengths, and waves of two tiles round the output alone to bf16;
 * the shapes beside the ranges bit-identical to the path that serves them;
 * 17 to 64 rows need no workspace (q3a_paged_decode_workspace_bytes of split_tokens 0 is 0) and so write none, whatever
   buffer the call is handed: a caller may share it between streams.
@@ -36,8 +37,9 @@ def _ctx(B, cap, kind):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["ragged", "full", "lone"])
-@pytest.mark.parametrize("B,cap", [(5, 272), (5, 2048), (16, 1040), (17, 528), (32, 1040), (33, 544), (63, 1024), (64, 2048)])
-def test_balanced_vs_oracle_and_append(cuda_device, B, cap, kind):
+@pytest.mark.parametrize("B,cap", [(5, 272), (5, 2048), (6, 768), (8, 512), (16, 272), (16, 1040), (16, 2048), (17, 528),
+                                   (32, 1040), (33, 544), (63, 1024), (64, 2048)])
+def test_small_batches_vs_oracle_and_append(cuda_device, B, cap, kind):
     ctx = _ctx(B, cap, kind)
     wl = W.make_decode("bal", cuda_device, ctx=ctx, num_pages=2 * B * (cap // 16 + 1), max_ctx=cap, seed=B + cap)
     L = wl.layers[0]
@@ -64,15 +66,16 @@ def test_balanced_vs_oracle_and_append(cuda_device, B, cap, kind):
 
 
 @pytest.mark.gpu
-def test_balanced_rope_form_exact_rows(cuda_device):
+@pytest.mark.parametrize("B", [12, 20])
+def test_rope_form_exact_rows(cuda_device, B):
     dev = cuda_device
-    ctx = _ctx(20, 1024, "ragged")
+    ctx = _ctx(B, 1024, "ragged")
     wl = W.make_decode("bal_rope", dev, ctx=ctx, num_pages=4096, max_ctx=1024, seed=7)
     rng = np.random.default_rng(5)
     r = lambda x: ora.bf16_round(np.asarray(x, np.float32))
     t = lambda x: torch.from_numpy(np.ascontiguousarray(x, np.float32)).to(dev).to(torch.bfloat16)
-    q, k = (r(rng.choice([-1.0, 1.0], size=(20, h, W.HEAD_DIM))) for h in (W.HQ, W.HKV))
-    v = r(rng.standard_normal((20, W.HKV, W.HEAD_DIM)))
+    q, k = (r(rng.choice([-1.0, 1.0], size=(B, h, W.HEAD_DIM))) for h in (W.HQ, W.HKV))
+    v = r(rng.standard_normal((B, W.HKV, W.HEAD_DIM)))
     qn, kn = (r(rng.uniform(0.5, 1.5, W.HEAD_DIM)) for _ in range(2))
     cos_t, sin_t = ora.rope_tables(1024)
     pos = np.maximum(ctx - 1, 0)
@@ -85,6 +88,33 @@ def test_balanced_rope_form_exact_rows(cuda_device):
                                           L.block_table, wl.scale, 0.0)
     ref = q3attn.paged_decode_append(t(qq), t(kk), t(v), kc, vc, old, L.block_table, wl.scale)
     assert torch.equal(out, ref) and torch.equal(kc, wl.k_cache) and torch.equal(vc, wl.v_cache)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,cap", [(6, 768), (16, 272), (12, 1280), (16, 2048), (20, 1024)])
+def test_a_row_does_not_depend_on_its_neighbours(cuda_device, B, cap):
+    wl = W.make_decode("bal_nb", cuda_device, ctx=_ctx(B, cap, "ragged"), num_pages=2 * B * (cap // 16 + 1), max_ctx=cap, seed=B)
+    L = wl.layers[0]
+    run = lambda lens: q3attn.paged_decode(L.q, wl.k_cache, wl.v_cache, lens, L.block_table, wl.scale)
+    out = run(wl.cache_seqlens)
+    for other in (0, 17, cap // 2 + 3, cap):
+        lens = wl.cache_seqlens.clone()
+        lens[1::2] = other
+        assert torch.equal(run(lens)[::2], out[::2]), other
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,cap", [(6, 768), (16, 272), (16, 1280)])
+def test_listed_chunks_round_the_output_alone(cuda_device, B, cap):
+    """q, k and v are exact in bf16 and the probabilities stay in fp32, so an output is within half a unit in the last place
+    (2^-8 of it) of the float64 result, but for the fp32 sums: 128 products of a score (about 1e-6 of p each) and the
+    tokens' sum, 2e-5 at the outputs' scale.  Probabilities rounded to bf16 are 7e-4 of the outputs' root mean square off."""
+    wl = W.make_decode("bal_p", cuda_device, ctx=_ctx(B, cap, "ragged"), num_pages=2 * B * (cap // 16 + 1), max_ctx=cap, seed=cap)
+    L = wl.layers[0]
+    out = to_np(q3attn.paged_decode(L.q, wl.k_cache, wl.v_cache, wl.cache_seqlens, L.block_table, wl.scale)).astype(np.float64)
+    ref = np.asarray(decode_oracle(wl, acc=np.float64), np.float64)
+    over = np.abs(out - ref) - (2.0 ** -8 * np.abs(ref) + 2e-5)
+    assert over.max() <= 0, over.max()
 
 
 ROW, CHUNKS, SK = q3attn.DECODE_ROW, q3attn.DECODE_CHUNKS, q3attn.DECODE_STREAMK
@@ -130,20 +160,10 @@ def test_no_workspace_is_touched_from_17_rows(cuda_device, B, cap):
 
 
 def test_workspace_query():
-    """5 to 16 rows: the records of 128-token chunks; 17 to 64 rows of up to 2,048 tokens: none, for every head count."""
+    """Up to 16 rows: the records of 128-token chunks; 17 to 64 rows of up to 2,048 tokens: none, for every head count."""
     ws = lambda B, pages, split, hkv=8: _lib.lib().q3a_paged_decode_workspace_bytes(B, 2 * hkv, hkv, 128, pages, 16, split)
     assert ws(16, 128, 0) == 16 * 16 * 8 * 1040 and ws(5, 17, 0) == 5 * 3 * 8 * 1040
     for B in (17, 32, 33, 64):
         for pages in (9, 16, 17, 33, 65, 128):
             for hkv in (1, 8, 16):
                 assert ws(B, pages, 0, hkv) == 0
-
-
-def test_chunk_count_arithmetic():
-    """ceil(n / d) as the kernel forms it, (n + d - 1/2) * rcp(d) truncated, with rcp off by one step either way."""
-    d = np.arange(1, 8193, dtype=np.int64)[:, None]
-    rcp = (np.float32(1) / d.astype(np.float32)).astype(np.float32)
-    for n in range(0, 8193, 61):
-        x = np.float32(n) + d.astype(np.float32) - np.float32(0.5)
-        for r in (rcp, np.nextafter(rcp, np.float32(0)), np.nextafter(rcp, np.float32(2))):
-            assert np.array_equal((x * r).astype(np.int64), -(-n // d)), n
