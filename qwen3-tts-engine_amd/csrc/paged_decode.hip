@@ -1580,14 +1580,13 @@ void paged_decode_row_kernel(const DecodeArgs a) {
   const int lane = threadIdx.x & 63;
   const int grp = lane >> 4;
   const int dl = (lane & 15) * 8;
-  const int CT = W * a.row_per;  // tiles per chunk (the one-launch path: the whole table)
-  const int cap = a.max_pages * a.page_size;
   int b = blockIdx.y, ch = blockIdx.z;
   if constexpr (kListed) {
     if (b >= a.batch) {
+      constexpr int CT = 2 * kListedWaves;
       const int extra = b - a.batch;  // this workgroup's place among the rows' chunks 1, 2, ...
       const int c = a.seqlens[min(lane, a.batch - 1)];
-      const int n = lane < a.batch ? (ctx_of<kAppend>(c, cap) + kTile - 1) / kTile : 0;
+      const int n = lane < a.batch ? (ctx_of<kAppend>(c, a.max_pages * a.page_size) + kTile - 1) / kTile : 0;
       const int more = n > CT ? (n + CT - 1) / CT - 1 : 0;  // row `lane`'s chunks past its first
       const int incl = wave_scan_incl(more);
       if (extra >= readlane(incl, 63)) return;  // uniform over the workgroup
@@ -1595,7 +1594,8 @@ void paged_decode_row_kernel(const DecodeArgs a) {
       ch = 1 + extra - (readlane(incl, b) - readlane(more, b));
     }
   }
-  const int tb = ch * CT;  // first tile of this workgroup's chunk
+  const int CT = W * a.row_per;  // tiles per chunk (the one-launch path: the whole table)
+  const int tb = ch * CT;        // first tile of this workgroup's chunk
 
   // Every load that does not depend on the context goes out together with the row's cache_seqlens entry: the
   // table entry of this lane's tile, q, (append form) the new k/v rows, (norm/rope form) the weights and cos/sin.
@@ -1606,6 +1606,7 @@ void paged_decode_row_kernel(const DecodeArgs a) {
                    "s"(a.q), "s"(a.q_sb), "s"(a.q_sh), "s"(a.scale_log2), "s"(a.kc), "s"(a.vc), "s"(a.kv_sp),
                    "s"(a.kv_st), "s"(a.kv_sh));
   const int c_row = a.seqlens[b];
+  const int cap = a.max_pages * a.page_size;
   const int t = kTile * (tb + w + lane * W);  // first token of this lane's tile
   const int pidx = min(t, cap - 1) / a.page_size;
   const int page = a.bt[(int64_t)b * a.bt_sb + pidx];
@@ -1728,43 +1729,19 @@ void paged_decode_row_kernel(const DecodeArgs a) {
   // Wave 0: lane -> (head h = lane / 32, dims 4*(lane%32)..+4), merging the W states.
   const int h = lane >> 5;
   const int d0 = (lane & 31) * 4;
-  // Each group's LDS reads are all in flight before the first is used, those of absent waves (inside the array, never
-  // used) among them; a loop over the W states waited for two LDS latencies each.
-  constexpr int kU = kListed ? kListedWaves : 8;
+  // One state at a time: the reads of eight states in flight ahead of their use unroll to code that makes small calls
+  // slower (8 rows log-uniform in [64, 272], norm/rope form: 8.63 -> 8.81 us per call).
   float M = kMaxSeed;
-#pragma unroll
-  for (int v0 = 0; v0 < kWaves; v0 += kU) {
-    if (v0 >= W) break;
-    float mv[kU];
-#pragma unroll
-    for (int u = 0; u < kU; ++u) mv[u] = rec[v0 + u][kG * kD + h];
-#pragma unroll
-    for (int u = 0; u < kU; ++u) M = v0 + u < W ? fmaxf(M, mv[u]) : M;
-  }
+  for (int v = 0; v < W; ++v) M = fmaxf(M, rec[v][kG * kD + h]);
   float Ls = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int v0 = 0; v0 < kWaves; v0 += kU) {
-    if (v0 >= W) break;
-    float mv[kU], lv[kU];
-    uint4 x[kU];
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const float* r = rec[v0 + u];
-      mv[u] = r[kG * kD + h];
-      lv[u] = r[kG * kD + kG + h];
-      x[u] = ld16(r + h * kD + d0);
-    }
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      if (v0 + u < W) {
-        const float wgt = fast_exp2(mv[u] - M);
-        Ls += lv[u] * wgt;
-        o[0] += __uint_as_float(x[u].x) * wgt;
-        o[1] += __uint_as_float(x[u].y) * wgt;
-        o[2] += __uint_as_float(x[u].z) * wgt;
-        o[3] += __uint_as_float(x[u].w) * wgt;
-      }
-    }
+  for (int v = 0; v < W; ++v) {
+    const float wgt = fast_exp2(rec[v][kG * kD + h] - M);
+    Ls += rec[v][kG * kD + kG + h] * wgt;
+    const uint4 x = ld16(&rec[v][h * kD + d0]);
+    o[0] += __uint_as_float(x.x) * wgt;
+    o[1] += __uint_as_float(x.y) * wgt;
+    o[2] += __uint_as_float(x.z) * wgt;
+    o[3] += __uint_as_float(x.w) * wgt;
   }
   if (nch > 1) {
     // Chunked form, a row spread over several chunks: this chunk's record, [kG][kD] o then m[kG], l[kG] (fp32).
