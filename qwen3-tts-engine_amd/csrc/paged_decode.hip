@@ -88,6 +88,7 @@ struct DecodeArgs {
   int* plan_claim;       // planned calls: one flag per range, set by the workgroup that takes it (zero between calls)
   int batch, hkv, split_tokens, max_splits, grid;
   int row_per;          // row-parallel path: tiles per wave of the table capacity (the host picks the kernel)
+  int row_slots;        // row-parallel path: rows that fill the CUs once, 0: rows in index order
   float scale_log2;
   // Norm/rope form (kRope instantiations): q and the new k rows arrive raw and are normalised and rotated in the
   // kernel (qk_norm_rope16/64): RMSNorm weights [kD] bf16, each row's RoPE cos/sin [kD] bf16 at row stride rs_sb.
@@ -1540,6 +1541,8 @@ __global__ __launch_bounds__(1024) void paged_decode_split_combine_kernel(const 
 constexpr int kMaxRowTiles = kOneSplitTokens / kTile;
 constexpr int kRowMaxWaves = 16;
 constexpr int kRowMaxPer = 8;             // rows of up to kRowMaxWaves * kRowMaxPer tiles = 2,048 tokens
+constexpr int kRowKeyBits = 14;           // a length in tiles (up to kRowMaxWaves * kRowMaxPer) and a row of 64
+static_assert(kRowMaxWaves * kRowMaxPer * 64 + 63 < 1 << kRowKeyBits, "a key has kRowKeyBits bits");
 constexpr int kRowMaxBatch = 64;            // beyond, stream-K (equal at 128-256 rows, ahead when ragged)
 constexpr int kRowRec = kG * kD + 2 * kG;  // floats per wave state: acc[kG][kD], m[kG], l[kG]
 // With several tiles per wave a workgroup has 8 waves of up to 16 tiles, and two workgroups share a CU: the new token's
@@ -1563,6 +1566,27 @@ constexpr int kChunkMax = 16;  // records per (row, KV head): the combine loads 
 // and a ballot, one more trip, or exit past the last one.  The chunks are cut from each row alone, so a row's result does not
 // depend on its neighbours.
 constexpr int kListedWaves = 4;
+
+// The row taken by grid place `at` where two workgroups share some CUs (S rows fill the CUs once, S < batch <= 2S <= 128,
+// batch <= 64): places at and S + at land on one CU, so the rows past S go to the CUs of the shorter ones, the shortest
+// beside the longest of them, and the longest rows have a CU alone.  Ranks by length, ties by index: lane i holds row
+// i's key, and the key of rank r is the largest that more than r keys reach, found bit by bit with ballots.  In index order
+// two long rows may meet on a CU (a CU streams two rows no faster than one after the other) while others idle.
+template <bool kAppend>
+__device__ __forceinline__ int row_by_rank(const DecodeArgs& a, int at, int S, int lane) {
+  const int c = a.seqlens[min(lane, a.batch - 1)];
+  const int n = (ctx_of<kAppend>(c, a.max_pages * a.page_size) + kTile - 1) / kTile;
+  const int key = lane < a.batch ? n * 64 + 63 - lane : -1;
+  const int m = a.batch - S;
+  const int rank = at < m ? S - m + at : (at < S ? at - m : S + m - 1 - (at - S));
+  int t = 0;
+#pragma unroll
+  for (int bit = kRowKeyBits - 1; bit >= 0; --bit) {
+    const int u = t | (1 << bit);
+    t = __builtin_popcountll(__ballot(key >= u)) > rank ? u : t;
+  }
+  return 63 - (t & 63);
+}
 
 template <bool kAppend, bool kMulti, bool kRope = false, bool kListed = false>
 __global__ __launch_bounds__(64 * (kListed ? kListedWaves : row_max_waves(kMulti)), kListed ? 4 : 1)
@@ -1593,6 +1617,9 @@ void paged_decode_row_kernel(const DecodeArgs a) {
       b = __builtin_popcountll(__ballot(incl <= extra));
       ch = 1 + extra - (readlane(incl, b) - readlane(more, b));
     }
+  }
+  if constexpr (kMulti && !kListed) {
+    if (a.row_slots > 0) b = row_by_rank<kAppend>(a, b, a.row_slots, lane);
   }
   const int CT = W * a.row_per;  // tiles per chunk (the one-launch path: the whole table)
   const int tb = ch * CT;        // first tile of this workgroup's chunk
@@ -1912,6 +1939,19 @@ bool chunk_geometry(int64_t cap_tiles, int* W, int* per, int* nch) {
 // Batches up to which long rows take the chunked form, and the table capacity (tiles) from which they do.
 constexpr int kChunkMaxBatch = 16;
 constexpr int kChunkMinTiles = 2 * kMaxRowTiles;
+
+// Rows in the order of their lengths (row_by_rank) where they fill the CUs more than once and at most twice: S rows, 0 for
+// index order.  Needs a lane a row, and tables of more than two tiles a wave: shorter ones have nothing to even out.
+// Us per call in a graph of 28, norm/rope form, one workgroup a CU and row fastest / two in index order / two by rank:
+//   tables of 2,048 tokens: 64 rows log-uniform in [64, 2048] 45.1 / 39.7 / 35.4, U[1024, 2048] 72.9 / 73.1 / 68.8; 56 rows
+//     of which 7 full 33.3 / 50.9 / 30.4; 36 x U[1024, 2048] 47.7 / 56.9 / 43.2; 40 x U[20, 200] 12.5 / 11.5 / 10.4
+//   272: 64 x U[136, 272] 16.9 / 14.9 / 15.0, 40 of which 5 full 12.7 / 10.9 / 9.4
+//   the cost of sharing a CU: rows of one length (within 5 %) that are long and little more than fill the CUs, 36 x
+//     U[1946, 2048] 60.4 / 65.8 / 65.5 (plain form up to +12 %; 44 rows +4 %, from 52 on +2 % at most)
+int row_slots(int batch, int hkv, int row_per) {
+  const int S = num_cus() / hkv;
+  return row_per > 2 && batch > S && batch <= 2 * S && batch <= 64 ? S : 0;
+}
 
 // Small batches of 256-token tables: two tiles a wave are one launch of the row kernel.
 constexpr int kRowOneTiles = 16;
@@ -2358,6 +2398,7 @@ static int launch_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
   a.ws = static_cast<float*>(workspace);
   if (row || chunks) {
     a.row_per = chunks ? chunk_per : (cap_tiles + row_waves - 1) / row_waves;
+    a.row_slots = row ? row_slots(batch, num_kv_heads, a.row_per) : 0;
     const bool listed = chunks && listed_chunks(batch, num_kv_heads, row_waves, chunk_per, nchunks);
     if (listed) {
       row_waves = kListedWaves;

@@ -117,6 +117,32 @@ def test_listed_chunks_round_the_output_alone(cuda_device, B, cap):
     assert over.max() <= 0, over.max()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("hkv,B,cap", [(8, 33, 272), (8, 40, 1040), (8, 63, 2048), (8, 64, 528), (16, 17, 272), (16, 20, 1040),
+                                       (16, 32, 2048), (5, 60, 528), (4, 64, 528)])
+def test_rows_in_the_order_of_their_lengths(cuda_device, hkv, B, cap):
+    """A batch whose rows fill the CUs more than once goes in the order of the lengths: each row as in a call of a few rows
+    (index order), ties, empty rows and rows past the capacity among them, in the plain and in the append form."""
+    g = torch.Generator(device=cuda_device).manual_seed(B)
+    pages = B * (cap // 16)
+    rnd = lambda *s: torch.randn(s, generator=g, device=cuda_device).to(torch.bfloat16)
+    kc, vc, q = rnd(pages, 16, hkv, 128), rnd(pages, 16, hkv, 128), rnd(B, 2 * hkv, 128)
+    k, v = rnd(B, hkv, 128), rnd(B, hkv, 128)
+    bt = torch.randperm(pages, generator=g, device=cuda_device).view(B, -1).to(torch.int32)
+    ctx = _ctx(B, cap, "ragged")
+    ctx[5:9] = [cap, cap, cap + 9, 17]
+    few = lambda f: torch.cat([f(slice(i, min(i + 8, B))) for i in range(0, B, 8)])
+    for lens in (ctx, np.full(B, cap // 2), np.where(np.arange(B) == B - 1, cap, 0)):
+        sl = torch.from_numpy(lens).to(torch.int32).to(cuda_device)
+        out = q3attn.paged_decode(q, kc, vc, sl, bt, 0.1)
+        assert torch.equal(out, few(lambda r: q3attn.paged_decode(q[r], kc, vc, sl[r], bt[r], 0.1, q3attn.DECODE_ROW)))
+        c1 = (kc.clone(), vc.clone())
+        app = q3attn.paged_decode_append(q, k, v, kc, vc, sl, bt, 0.1)
+        assert torch.equal(app, few(lambda r: q3attn.paged_decode_append(q[r], k[r], v[r], *c1, sl[r], bt[r], 0.1,
+                                                                         q3attn.DECODE_ROW)))
+        assert torch.equal(kc, c1[0]) and torch.equal(vc, c1[1])
+
+
 ROW, CHUNKS, SK = q3attn.DECODE_ROW, q3attn.DECODE_CHUNKS, q3attn.DECODE_STREAMK
 
 
