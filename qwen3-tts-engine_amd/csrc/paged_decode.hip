@@ -1547,8 +1547,7 @@ constexpr int kRowMaxBatch = 64;            // beyond, stream-K (equal at 128-25
 constexpr int kRowRec = kG * kD + 2 * kG;  // floats per wave state: acc[kG][kD], m[kG], l[kG]
 // With several tiles per wave a workgroup has 8 waves of up to 16 tiles, and two workgroups share a CU: the new token's
 // swap is pinned ahead of the tile's arithmetic, which keeps the append forms at 116 registers (147 left to itself: one
-// workgroup a CU).  64 rows log-uniform in [64, 1200]: 30.2 -> 25.2 us per call with the head-fastest grid; 20 rows of
-// up to 60 tokens in 256-token tables, 16 waves of one tile -> 8 of two: 8.1 -> 5.7.
+// workgroup a CU).  64 rows log-uniform in [64, 1200]: 30.2 -> 25.2 us per call with the head-fastest grid.
 constexpr int row_max_waves(bool multi) { return multi ? kRowMaxWaves / 2 : kRowMaxWaves; }
 
 //
@@ -1588,8 +1587,9 @@ __device__ __forceinline__ int row_by_rank(const DecodeArgs& a, int at, int S, i
   return 63 - (t & 63);
 }
 
-template <bool kAppend, bool kMulti, bool kRope = false, bool kListed = false>
-__global__ __launch_bounds__(64 * (kListed ? kListedWaves : row_max_waves(kMulti)), kListed ? 4 : 1)
+// kPair: two tiles a wave, the probabilities in fp32 (all listed chunks, and the row path's tables of two tiles a wave).
+template <bool kAppend, bool kMulti, bool kRope = false, bool kListed = false, bool kPair = kListed>
+__global__ __launch_bounds__(64 * (kListed ? kListedWaves : row_max_waves(kMulti)), kPair ? 4 : 1)
 void paged_decode_row_kernel(const DecodeArgs a) {
   static_assert(kAppend || !kRope, "the norm/rope form is an append form");
   constexpr int kWaves = kListed ? kListedWaves : kRowMaxWaves;
@@ -1618,7 +1618,7 @@ void paged_decode_row_kernel(const DecodeArgs a) {
       ch = 1 + extra - (readlane(incl, b) - readlane(more, b));
     }
   }
-  if constexpr (kMulti && !kListed) {
+  if constexpr (kMulti && !kPair) {
     if (a.row_slots > 0) b = row_by_rank<kAppend>(a, b, a.row_slots, lane);
   }
   const int CT = W * a.row_per;  // tiles per chunk (the one-launch path: the whole table)
@@ -1704,13 +1704,19 @@ void paged_decode_row_kernel(const DecodeArgs a) {
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    tile_update<kListed>(a, L, q, T, j, grp, m, l, acc);
+    tile_update<kPair>(a, L, q, T, j, grp, m, l, acc);
   };
 
   if constexpr (!kMulti) {
     KVTile A;
     issue(0, A);
     consume(A, 0);
+  } else if constexpr (kPair && !kRope) {  // (the norm/rope form would spill here)
+    KVTile A, Bt;
+    issue(0, A);
+    issue(1, Bt);
+    consume(A, 0);
+    if (L.n > 1) consume(Bt, 1);
   } else {
     KVTile A, Bt;
     issue(0, A);
@@ -1953,15 +1959,18 @@ int row_slots(int batch, int hkv, int row_per) {
   return row_per > 2 && batch > S && batch <= 2 * S && batch <= 64 ? S : 0;
 }
 
-// Small batches of 256-token tables: two tiles a wave are one launch of the row kernel.
-constexpr int kRowOneTiles = 16;
+// Tables of 9 to 16 tiles: 8 waves of two tiles with the probabilities in fp32 (kPair), in place of a wave a tile; up to
+// 16 rows of them too, in one launch in place of chunks and their combine.  Us per call in a graph of 28, before / now:
+//   norm/rope, rows log-uniform in [64, 256]: 8 rows 8.6 / 7.9, 24 rows 9.5 / 8.5, 64 rows 18.3 / 12.8; 64 in [64, 144] 13.8 / 11.1
+//   plain: 8 rows 7.7 / 6.4, 64 rows 12.4 / 10.8; 24 in [64, 144] 6.5 / 6.1
+constexpr int kRowOneTiles = kRowMaxWaves;
 
 // The listed form takes the place of 8-wave workgroups of 128-token chunks (tables up to 2,048 tokens) where their grid
 // of the table's capacity is more than one workgroup a CU and each row has a lane: below, the workgroups of absent chunks are
 // on CUs of their own, and the extra trip shows.  Us per call in a graph of 28, chunks of the capacity / listed:
-//   norm/rope: 8 x 512 (256 workgroups) 9.1 / 9.1 log-uniform, 9.0 / 9.3 U[205, 358]; 6 x U[384, 768] (288) 11.4 / 9.6;
-//     16 rows log-uniform in [64, 1280] 20.2 / 12.8, U[1946, 2048] 33.1 / 30.0; all shapes from 288 workgroups 0.40 to 1.01
-//   plain: 16 log-uniform in [64, 1280] 15.3 / 12.1, 6 x U[1024, 2048] 13.4 / 13.9 (the worst), the rest 0.54 to 1.03
+//   norm/rope: 6 x U[384, 768] (288 workgroups) 11.4 / 9.3; 16 rows log-uniform in [64, 1280] 20.2 / 11.9, 16 x U[1946, 2048]
+//     33.1 / 29.7; all shapes from 288 workgroups 0.39 to 0.98; 8 x U[205, 358] of 512-token tables (256) 9.0 / 9.3
+//   plain: 10.0 / 8.5, 15.3 / 10.8, 27.9 / 27.8, 0.51 to 1.00, 8.2 / 8.4
 bool listed_chunks(int batch, int hkv, int row_waves, int row_per, int nchunks) {
   return row_waves == 8 && row_per == 1 && batch <= 64 && (int64_t)batch * nchunks * hkv > num_cus();
 }
@@ -2431,6 +2440,13 @@ static int launch_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
           hipLaunchKernelGGL((paged_decode_row_kernel<true, true, false, true>), rgrid, rblock, 0, st, a);
         else
           hipLaunchKernelGGL((paged_decode_row_kernel<false, true, false, true>), rgrid, rblock, 0, st, a);
+      } else if (row && a.row_per == 2) {
+        if (rope)
+          hipLaunchKernelGGL((paged_decode_row_kernel<true, true, true, false, true>), rgrid, rblock, 0, st, a);
+        else if (append)
+          hipLaunchKernelGGL((paged_decode_row_kernel<true, true, false, false, true>), rgrid, rblock, 0, st, a);
+        else
+          hipLaunchKernelGGL((paged_decode_row_kernel<false, true, false, false, true>), rgrid, rblock, 0, st, a);
       } else if (a.row_per == 1) {
         if (rope)
           hipLaunchKernelGGL((paged_decode_row_kernel<true, false, true>), rgrid, rblock, 0, st, a);
