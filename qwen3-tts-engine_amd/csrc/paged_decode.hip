@@ -1895,19 +1895,6 @@ int sk_grid_of(int hkv, int form) {
   return g;
 }
 
-// Compute units of the current device (cached per device).
-int num_cus() {
-  static std::atomic<int> cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int cus = cache[dev].load(std::memory_order_relaxed);
-  if (cus <= 0) {
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 256;
-    cache[dev].store(cus, std::memory_order_relaxed);
-  }
-  return cus;
-}
-
 int sk_grid(int hkv) {
   const int g0 = sk_grid_of(hkv, 0), g1 = sk_grid_of(hkv, 1), g2 = hkv <= 8 ? sk_grid_of(hkv, 2) : 0;
   return std::max(g0, std::max(g1, g2));

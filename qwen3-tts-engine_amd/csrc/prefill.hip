@@ -1312,7 +1312,7 @@ static int resident_slots() {
 //   dense (every query tile sees the prefix): 8 x 100 + 50 8.3 / 9.9, 1 x 200 + 100 11.4 / 10.6, 4 x 250 + 150 14.9 / 12.9,
 //     6 x 210 + 170 (two teams) 14.8 / 13.6; two teams below that: 4 x U[150, 400] packed 13.3 / 12.9, 8 x U[150, 250] 18.4 / 19.6
 static int key_split(int num_seqs, int hkv, int max_seqlen_q, bool dense, int seqlen_k) {
-  const int cus = resident_slots() / 3;
+  const int cus = num_cus();
   const int64_t heads = (int64_t)num_seqs * hkv;
   const int keys = dense ? seqlen_k : max_seqlen_q;
   if (keys >= (dense ? 288 : 384) && heads * ((max_seqlen_q + 31) / 32) <= cus) return 4;

@@ -305,4 +305,8 @@ __device__ __forceinline__ uint32_t qk_norm_rope64(uint32_t x, uint32_t w, uint3
 namespace q3a {
 // Records a message for q3a_last_error() on this thread and returns `code`.
 int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
+
+// Compute units of the current device (cached per device; two host threads may fill an entry at once, both with the same
+// value).
+int num_cus();
 }  // namespace q3a
