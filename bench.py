@@ -294,8 +294,8 @@ def make_planned_frame(wl, bts):
 
 
 def decode_kernel_name(wl, split, planned=False):
-    """The kernels one decode call of this workload launches (the library needs no workspace exactly when it takes
-    the row-parallel path, for split 0)."""
+    """The kernels one decode call of this workload launches (for split 0 the library takes the row-parallel path where it
+    needs no workspace, and for up to 16 rows of 256-token tables)."""
     from q3attn import _lib
 
     if planned:
@@ -307,7 +307,8 @@ def decode_kernel_name(wl, split, planned=False):
                                                            L.block_table.shape[1], wl.page_size, code)
     if split > 0:
         return "paged decode call (fixed-split decode kernel + combine kernel)"
-    if split == -1 or (split == 0 and ws(0) == 0):
+    one_launch = ws(0) == 0 or (wl.batch <= 16 and L.block_table.shape[1] * wl.page_size <= 256)
+    if split == -1 or (split == 0 and one_launch):
         return "paged decode call (row-parallel kernel, one launch)"
     if split == -2 or (split == 0 and ws(0) == ws(-2)):
         return "paged decode call (chunked decode kernel + chunk combine kernel)"
