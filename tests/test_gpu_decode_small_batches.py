@@ -159,6 +159,41 @@ def test_shapes_beside_its_range(cuda_device, B, cap, path):
     assert torch.equal(out, forced)
 
 
+@pytest.mark.gpu
+def test_batches_past_the_grid_limit(cuda_device):
+    """Narrow tables with more rows than a grid dimension holds (65,535) go in slices of rows: the rows around the cut and the
+    last one as in a call of those rows alone, plain, append and norm/rope form, and the slots that they wrote."""
+    B, dev = 65600, cuda_device
+    g = torch.Generator(device=dev).manual_seed(65)
+    rnd = lambda *s: torch.randn(s, generator=g, device=dev, dtype=torch.bfloat16)
+    kc, vc = rnd(B, 16, 8, 128), rnd(B, 16, 8, 128)
+    qkv, qn, kn, cos, sin = rnd(B, 32 * 128), rnd(128), rnd(128), rnd(B, 128), rnd(B, 128)
+    q, k, v = qkv[:, :2048].view(B, 16, 128), qkv[:, 2048:3072].view(B, 8, 128), qkv[:, 3072:].view(B, 8, 128)
+    bt = torch.randperm(B, generator=g, device=dev).to(torch.int32).view(B, 1)
+    lens = torch.randint(0, 16, (B,), generator=g, device=dev, dtype=torch.int32)
+    r = torch.tensor([0, 1, 65533, 65534, 65535, 65536, 65537, B - 2, B - 1], device=dev)
+    pages = bt[r, 0].long()
+
+    def forms(x):
+        pools = [(kc.clone(), vc.clone()) for _ in range(2)] if x is not None else [(kc, vc)] * 2
+        s = (lambda t: t[x]) if x is not None else (lambda t: t)
+        return (q3attn.paged_decode(s(q), kc, vc, s(lens), s(bt), 0.1),
+                lambda: (q3attn.paged_decode_append(s(q), s(k), s(v), *pools[0], s(lens), s(bt), 0.1), *pools[0]),
+                lambda: (q3attn.paged_decode_append_rope(s(q), s(k), s(v), qn, kn, s(cos), s(sin), *pools[1], s(lens), s(bt), 0.1,
+                                                         1e-6), *pools[1]))
+
+    few = forms(r)
+    few = [few[0], few[1](), few[2]()]
+    clean = kc[pages].clone(), vc[pages].clone()
+    big = forms(None)
+    assert torch.equal(big[0][r], few[0])
+    for f, want in zip(big[1:], few[1:]):
+        out, pk, pv = f()
+        assert torch.equal(out[r], want[0])
+        assert torch.equal(pk[pages], want[1][pages]) and torch.equal(pv[pages], want[2][pages])
+        kc[pages], vc[pages] = clean
+
+
 def _c_decode(fn, wl, out, *ws):
     L = wl.layers[0]
     return fn(L.q.data_ptr(), L.q.stride(0), L.q.stride(1), wl.k_cache.data_ptr(), wl.v_cache.data_ptr(),
