@@ -15,6 +15,7 @@ import q3attn
 from helpers import to_np
 from oracle import attention as ora
 from q3attn import workloads as W
+from test_gpu_prefill_append import _run_both, _table
 
 pytestmark = pytest.mark.gpu
 
@@ -147,3 +148,31 @@ def test_a_loose_bound_takes_the_same_kernel(cuda_device, lens, bound):
                                            True, 1e-6), *p, *r)
     for a, b in zip(forms(max(lens)), forms(bound)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("lens,prefix", [([400], [37]), ([384, 100], [32, 50]),      # four teams
+                                         ([384, 353, 5], [0, 45, 300]), ([1057], [3])])  # two
+def test_packed_append_after_a_prefix(cuda_device, lens, prefix, causal):
+    """Keys before the first query (a multiple of a tile or not), with and without the mask: the pool rows go out through the
+    prologue's copies, or from the stages of the last tiles.  Output and pool as in scatter + packed prefill, bit for bit,
+    and the output against the fp32 softmax."""
+    dev, g = cuda_device, torch.Generator().manual_seed(sum(lens))
+    Lq, Lk = np.array(lens), np.array(lens) + np.array(prefix)
+    cu_q, cu_k = (np.concatenate([[0], np.cumsum(x)]).astype(np.int32) for x in (Lq, Lk))
+    rnd = lambda n, h: torch.randn(n, h, 128, generator=g).to(torch.bfloat16).to(dev)
+    q, k, v = rnd(cu_q[-1], 16), rnd(cu_k[-1], 8), rnd(cu_k[-1], 8)
+    P = -(-int(Lk.max()) // 16)
+    out, _, _, n = _run_both(dev, q, k, v, cu_q, cu_k, int(Lq.max()), _table(len(lens), P, 4 * P * len(lens), False, 7), 16,
+                             4 * P * len(lens), 0.09, causal)
+    assert n == Lq.sum()
+    qf, kf, vf = to_np(q), to_np(k), to_np(v)
+    ref = np.zeros_like(qf)
+    for s in range(len(lens)):
+        r, c = slice(cu_q[s], cu_q[s + 1]), slice(cu_k[s], cu_k[s + 1])
+        see = np.arange(Lk[s])[None, :] <= (prefix[s] + np.arange(Lq[s])[:, None] if causal else Lk[s])
+        for h in range(16):
+            a = np.where(see, qf[r, h] @ kf[c, h // 2].T * 0.09, -np.inf)
+            p = np.exp(a - a.max(-1, keepdims=True))
+            ref[r, h] = (p / p.sum(-1, keepdims=True)) @ vf[c, h // 2]
+    check(out, ref, f"packed {lens} after {prefix}, causal {causal}")
