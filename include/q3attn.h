@@ -76,12 +76,10 @@ const char* q3a_last_error(void);
  * no tokens.  Requirements: D == 128, Hq == 2*Hkv, 1 <= Hkv <= 16, page_size % 16 == 0,
  * 16-byte aligned rows.  split_tokens == 0 lets the library choose the decomposition from the batch and
  * the table capacity max_pages_per_seq*page_size (never from the device-resident lengths): tables of at most
- * 128 tokens and batches of 17 to 64 rows with tables of at most 2,048 tokens take Q3A_DECODE_ROW, longer tables of at most
- * 16 rows Q3A_DECODE_CHUNKS; of these, tables of 256 tokens take the one-launch kernel all the same (with the workspace of
- * the chunks) and 5 to 16 rows of tables up to 2,048 tokens are cut into chunks on the device from the rows' lengths, so
- * that they fill it once (the balanced form, in the same workspace).  Larger batches take stream-K (a persistent grid
- * sized to the device, balanced over all rows' 16-token tiles; batch <= 4096,
- * larger batches fall back to q3a_paged_decode_default_split()).  The path codes above force one of them;
+ * 128 tokens and batches of at most 64 rows with tables of at most 2,048 tokens take Q3A_DECODE_ROW, except batches of
+ * at most 16 rows with tables of 256 tokens or more, which take Q3A_DECODE_CHUNKS (tables of 256 tokens are one launch
+ * of the row kernel all the same, and ask for the workspace of the chunks).  Larger batches take stream-K (a persistent
+ * grid sized to the device, balanced over all rows' 16-token tiles; batch <= 4096, larger batches fall back to q3a_paged_decode_default_split()).  The path codes above force one of them;
  * split_tokens > 0 (a multiple of 16, <= 1024) selects one workgroup per (row, split of that many tokens).
  */
 int q3a_paged_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h,

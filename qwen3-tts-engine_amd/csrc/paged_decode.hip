@@ -23,7 +23,7 @@
 // the same kind of combine.  Narrow tables (at most 128 tokens, small batches 256) and batches of at most 64 rows of
 // up to 2,048 tokens take the row-parallel kernel instead: one workgroup per (row, KV head), the row's tiles
 // spread over its waves and merged in LDS, one launch; or, where one such workgroup would be too long a chain or
-// too uneven a share, its chunked and balanced forms: chunks of each row, then a combine.
+// too uneven a share (at most 16 rows), its chunked form: chunks of each row, then a combine.
 //
 // Append form (flash_attn_with_kvcache with k=, v=; replaces the index_copy_ pair of
 // engine/talker.py:72-73 before the call at :77): cache_seqlens counts the tokens already cached,

@@ -340,17 +340,16 @@ void prefill_kernel(const PrefillArgs a) {
   const int wmax = wfirst >= Lq ? -1 : (a.causal ? min(Lk - 1, Lk - Lq + min(Lq - 1, wfirst + 15)) : Lk - 1);
 
   // Tile copies.  A 32-key tile is 2 groups of 16 keys and a group never straddles a page (page sizes are
-  // powers of two >= 16), so each group has one uniform base address; waves 0 and 1 copy K groups 0 and 1,
-  // waves 2 and 3 the V groups, with four direct-to-LDS loads each (instruction i: rows 4i..4i+3 of the group,
-  // 1 KiB).  The descriptor covers
-  // exactly the group's valid rows of head g: rows past the sequence and groups on an invalid page arrive as
-  // zeros.  Lane l of instruction i lands at LDS chunk slot l & 15 of row rr = 4i + (l >> 4), so it fetches
+  // powers of two >= 16), so each group has one uniform base address; the first half of a team's waves
+  // copies the K groups (one each of four waves, both of two), the second the V groups, with four direct-to-LDS loads a
+  // group (instruction i: rows 4i..4i+3 of the group, 1 KiB).  The descriptor covers exactly the group's valid rows of
+  // head g: rows past the sequence and groups on an invalid page arrive as zeros.  Lane l of instruction i lands at LDS chunk slot l & 15 of row rr = 4i + (l >> 4), so it fetches
   // global chunk (l & 15) ^ rr (V: ^ v_swz(rr)): the swizzle is applied on the global side.  Page ids come from a lane-wise
   // window (lane i = table entry pwin_base + i), read with v_readlane; it is refilled once per 64 pages.
   static_assert(kKT == 32, "the copy assignment below is for 2 groups per tile");
   constexpr int kGroupsPerWave = 4 / kQW;
   const int cgrp0 = wave & (kQW / 2 - 1);        // the 16-key group(s) of a tile this wave copies
-  const uint16_t* cbase = copies_k ? a.k : a.v;  // waves 0, 1 copy K; waves 2, 3 copy V
+  const uint16_t* cbase = copies_k ? a.k : a.v;
   auto group_rsrc = [&](const uint16_t* base, int t, int cgrp, int page) __attribute__((always_inline)) {
     const int j0 = t * kKT + 16 * cgrp;
     const int nv = min(16, Lk - j0);
@@ -794,7 +793,7 @@ __global__ __launch_bounds__(64 * (kRope ? kResRopeWaves : kResMaxGroups)) void 
   if (app && lane < min(kResMaxTiles * kKT / 16, a.p_max_pages)) pwo = a.pbt[(int64_t)s * a.pbt_sb + lane];
 
   // Copies: the 16-key groups of K and V (2 per tile and operand) are dealt round-robin to the waves; four
-  // direct-to-LDS loads each, same layout and swizzle as the tiled kernel.
+  // direct-to-LDS loads each, the tiled kernel's layout with K's swizzle (key & 15) on both operands.
   const int ngroups = 4 * ntiles;
   // The copies' kernel arguments (and the append form's table arguments) are read with the others, in one batch:
   // left to itself the compiler reads them after the first batch has returned, one more round trip before the first
