@@ -79,7 +79,8 @@ const char* q3a_last_error(void);
  * 128 tokens and batches of at most 64 rows with tables of at most 2,048 tokens take Q3A_DECODE_ROW, except batches of
  * at most 16 rows with tables of 256 tokens or more, which take Q3A_DECODE_CHUNKS (tables of 256 tokens are one launch
  * of the row kernel all the same, and ask for the workspace of the chunks).  Larger batches take stream-K (a persistent
- * grid sized to the device, balanced over all rows' 16-token tiles; batch <= 4096, larger batches fall back to q3a_paged_decode_default_split()).  The path codes above force one of them;
+ * grid sized to the device, balanced over all rows' 16-token tiles; batch <= 4096, larger batches fall back to
+ * q3a_paged_decode_default_split()).  The path codes above force one of them;
  * split_tokens > 0 (a multiple of 16, <= 1024) selects one workgroup per (row, split of that many tokens).
  */
 int q3a_paged_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h,

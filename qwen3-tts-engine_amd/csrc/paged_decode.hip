@@ -1566,9 +1566,9 @@ constexpr int kChunkMax = 16;  // records per (row, KV head): the combine loads 
 // depend on its neighbours.
 constexpr int kListedWaves = 4;
 
-// The row taken by grid place `at` where two workgroups share some CUs (S rows fill the CUs once, S < batch <= 2S <= 128,
-// batch <= 64): places at and S + at land on one CU, so the rows past S go to the CUs of the shorter ones, the shortest
-// beside the longest of them, and the longest rows have a CU alone.  Ranks by length, ties by index: lane i holds row
+// The row taken by grid place `at` where two workgroups share some CUs (S rows fill the CUs once, S < batch <= 2S,
+// batch <= 64): places at and S + at land on one CU (only the speed depends on it), so the rows past S go to the CUs of
+// the shorter ones, the shortest beside the longest of them, and the longest rows have a CU alone.  Ranks by length, ties by index: lane i holds row
 // i's key, and the key of rank r is the largest that more than r keys reach, found bit by bit with ballots.  In index order
 // two long rows may meet on a CU (a CU streams two rows no faster than one after the other) while others idle.
 template <bool kAppend>
